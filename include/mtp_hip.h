@@ -256,7 +256,9 @@ int mtp_attn_fwd_f32(const float* q, const float* k, const float* v, int64_t b, 
                      const int32_t* seg_id, const int32_t* seg_start, float* o, float* lse,
                      void* stream);
 
-/* Workspace bytes of mtp_attn_bwd_f32: the fp32 row term D [b][hq][s]. */
+/* Workspace bytes of mtp_attn_bwd_f32: the fp32 row term D [b][hq][s]; when the dK/dV pass splits its
+ * key blocks to fill the GPU, the fp32 partials [splits][2][b][hkv][s][dh] follow from the next 256-byte
+ * boundary. With less than that, but room for D, the pass runs unsplit. */
 size_t mtp_attn_bwd_f32_workspace_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t dh);
 
 /* fp32 backward, as mtp_attn_bwd; dq, dk, dv fp32. Replaces launch_bwd_D / launch_bwd_dq /

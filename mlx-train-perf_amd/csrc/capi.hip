@@ -528,9 +528,9 @@ int mtp_attn_fwd_f32(const float* q, const float* k, const float* v, int64_t b, 
 }
 
 size_t mtp_attn_bwd_f32_workspace_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t dh) {
-  (void)dh;
   if (b < 1 || hq < 1 || hkv < 1 || s < 1 || hq % hkv || b * hq * s > kMaxDim) return 0;
-  return (size_t)b * (size_t)hq * (size_t)s * sizeof(float);
+  const int ns = mtp::attn32_dkv_splits((int)b, (int)hq, (int)hkv, (int)s, (int)dh);
+  return mtp::attn32_bwd_workspace((int)b, (int)hq, (int)hkv, (int)s, (int)dh, ns);
 }
 
 int mtp_attn_bwd_f32(const float* q, const float* k, const float* v, const float* o, const float* lse, const float* d_o,
@@ -542,12 +542,15 @@ int mtp_attn_bwd_f32(const float* q, const float* k, const float* v, const float
   if (!o || !lse || !d_o || !d_q || !d_k || !d_v) return fail(MTP_ERR_INPUT, "o, lse, d_o, d_q, d_k, d_v must be non-null");
   if (!aligned16(o) || !aligned16(d_o) || !aligned16(d_q) || !aligned16(d_k) || !aligned16(d_v))
     return fail(MTP_ERR_UNSUPPORTED, "o, d_o, d_q, d_k, d_v must be 16-byte aligned");
-  const size_t need = mtp_attn_bwd_f32_workspace_bytes(b, hq, hkv, s, dh);
+  // D is all it needs; a workspace without room for the split's partials runs the dK/dV pass unsplit.
+  const size_t need = mtp::attn32_bwd_workspace((int)b, (int)hq, (int)hkv, (int)s, (int)dh, 1);
+  const bool split = workspace_bytes >= mtp_attn_bwd_f32_workspace_bytes(b, hq, hkv, s, dh);
   if (!workspace || workspace_bytes < need)
     return fail(MTP_ERR_WORKSPACE, "fp32 attention backward needs a workspace of %zu bytes (got %zu)", need, workspace ? workspace_bytes : (size_t)0);
   mtp::AttnShape sh{(int)b, (int)hq, (int)hkv, (int)s, (int)dh, scale, (int)causal};
+  const int ns = split ? mtp::attn32_dkv_splits(sh.b, sh.hq, sh.hkv, sh.s, sh.dh) : 1;
   hipError_t e = mtp::launch_attn32_bwd(sh, q, k, v, o, lse, d_o, seg_start, d_q, d_k, d_v,
-                                        static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+                                        static_cast<float*>(workspace), ns, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(MTP_ERR_RUNTIME, "fp32 attention backward launch failed: %s", hipGetErrorString(e));
   return ok();
 }

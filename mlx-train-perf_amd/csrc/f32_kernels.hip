@@ -438,286 +438,484 @@ __global__ __launch_bounds__(256) void lce32_dw_kernel(const float* __restrict__
 }
 
 // ------------------------------------------------------------------------------------------
-// Attention. A workgroup of 4 waves owns 128 positions of one head (queries: forward and dQ; keys
-// of one kv head: dK/dV); each wave 32 of them as its MFMA column block. 32-position tiles of the
-// other side go through LDS ([32][DH + pad] fp32; +4 keeps the 16-byte row-fragment reads on
-// distinct banks, +8 the transposed column reads of the two lane halves).
+// Attention on v_mfma_f32_16x16x4_f32 (lane l: col = l % 16, g = l / 16; it supplies A[col][g] and
+// B[g][col] and holds C[4 g + r][col], r < 4). A wave owns 16 positions of one head as the MFMA columns
+// (queries: forward and dQ; keys: dK/dV) and keeps their rows and gradients in registers; the 8 waves
+// of a workgroup share 32-position tiles of the other side, copied global -> LDS one tile ahead.
+//
+// The matrix pipe bounds it: a 16x16x4 product takes 32 cycles of its SIMD, so a forward tile is 4096
+// MFMA cycles per wave against 32 KiB of LDS reads and ~100 VALU instructions. 32-position waves on
+// tiles staged through registers between two barriers left most of it idle: at S = 2048 (16/4 heads,
+// head_dim 128, causal) one wave per SIMD waited at the barriers, and the 64 key blocks of dK/dV, of very
+// unequal work, were all that 256 CUs had. Hence 16-position waves, which need half the registers, and
+// a workgroup of two half-workgroups of 4 waves on two position blocks: under the causal mask the
+// mirrored pair (block p and block n - 1 - p), whose work adds up to the same for every pair, with one
+// wave of each on every SIMD; otherwise two adjacent blocks, which read the same tiles.
+// Measured there: forward 456 -> 177 us, dQ 570 -> 242, dK/dV 2537 -> 322 (4 splits and their sum), 97-109
+// TFLOP/s; at S = 8192, 32/8 heads 4.08, 6.19 and 8.13 ms, 133-135 of the 153 TFLOP/s a library fp32
+// matrix product reaches.
+//
+// Row reads (products over head_dim): lane (col, g) reads 16-byte chunks of row col, chunk order
+// row_chunk(c, g) -- the contraction may visit head_dim in any order as long as both operands do.
+// Column reads (products over the tile's positions): lane (col, g) reads chunk 16 b + col of row
+// 4 g + s, one read for four products, whose output rows are head_dims 64 b + 4 i + j (product j, row
+// i). Chunk k of row r sits at slot k ^ (r % 16): the 16 lanes of a g, and the lanes 0-7 / 32-39 of a
+// read, fall on distinct banks in both.
+//
 // Masks: key j visible to query i iff j < S, (causal) j <= i, (packed) seg_start[i] <= j; in the
 // packed layout (contiguous, ascending, gapless segments) that is "same segment and j <= i".
 // ------------------------------------------------------------------------------------------
-template <int DH>
-struct ALay {
-  static constexpr int kPr = DH + 4;  // rows read as 16-byte fragments (and columns)
-  static constexpr int kPc = DH + 8;  // rows read only as columns
-  static constexpr int kQuads = 32 * DH / 4;
-};
-// Copy rows [p0, p0 + 32) of a [S][DH] fp32 matrix into LDS with pitch P (rows past S as zeros).
-template <int DH, int P>
-__device__ __forceinline__ void tile_in(const float* __restrict__ src, int p0, int S, float* lds) {
-  for (int idx = threadIdx.x; idx < ALay<DH>::kQuads; idx += 256) {
-    const int row = idx / (DH / 4), c4 = idx % (DH / 4);
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-    if (p0 + row < S) x = *reinterpret_cast<const f32x4*>(src + (long)(p0 + row) * DH + 4 * c4);
-    *reinterpret_cast<f32x4*>(lds + row * P + 4 * c4) = x;
-  }
+constexpr int kPos = 32;  // positions per LDS tile
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-// This lane's half of a row as MFMA B-operand registers for the d contraction: x[8 c + s] =
-// row[16 c + 8 h + s].
-template <int DH>
-__device__ __forceinline__ void row_regs(const float* __restrict__ row, bool valid, float (&x)[DH / 2]) {
-  const int h = (threadIdx.x & 63) >> 5;
-#pragma unroll
-  for (int c = 0; c < DH / 16; ++c) {
-    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
-    if (valid) {
-      lo = *reinterpret_cast<const f32x4*>(row + 16 * c + 8 * h);
-      hi = *reinterpret_cast<const f32x4*>(row + 16 * c + 8 * h + 4);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      x[8 * c + s] = lo[s];
-      x[8 * c + 4 + s] = hi[s];
-    }
-  }
-}
-// acc (32 rows of the LDS tile x this lane's column) += tile rows . x over the d contraction.
-template <int DH, int P>
-__device__ __forceinline__ void dot_rows(const float* lds, const float (&x)[DH / 2], f32x16& acc) {
-  const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
-  const float* row = lds + i * P + 8 * h;
-#pragma unroll
-  for (int c = 0; c < DH / 16; ++c) {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(row + 16 * c);
-    const f32x4 hi = *reinterpret_cast<const f32x4*>(row + 16 * c + 4);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc = mfma2(lo[s], x[8 * c + s], acc);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc = mfma2(hi[s], x[8 * c + 4 + s], acc);
-  }
-}
-// out[db] (d x this lane's column) += tile^T . p over the tile's 32 rows, p[r] the weight of row
-// rrow(r, h) (an accumulator of the lane's column).
-template <int DH, int P>
-__device__ __forceinline__ void dot_cols(const float* lds, const f32x16& p, f32x16 (&out)[DH / 32]) {
-  const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
-#pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    const float* row = lds + rrow(s, h) * P + i;
-#pragma unroll
-    for (int db = 0; db < DH / 32; ++db) out[db] = mfma2(row[32 * db], p[s], out[db]);
-  }
-}
-// Writes acc (d x this lane's row q) * mul to out[q][d].
-template <int DH>
-__device__ __forceinline__ void store_rows(float* __restrict__ out, const f32x16 (&acc)[DH / 32], float mul) {
-  const int h = (threadIdx.x & 63) >> 5;
-#pragma unroll
-  for (int db = 0; db < DH / 32; ++db)
-#pragma unroll
-    for (int rq = 0; rq < 4; ++rq)
-      *reinterpret_cast<f32x4*>(out + 32 * db + 8 * rq + 4 * h) =
-          f32x4{acc[db][4 * rq] * mul, acc[db][4 * rq + 1] * mul, acc[db][4 * rq + 2] * mul, acc[db][4 * rq + 3] * mul};
+__device__ __forceinline__ void copies_landed() {
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
 }
 
-// Forward (DQ = false) and dQ (DQ = true): 128 queries of one head per workgroup, heaviest first.
-template <int DH, bool PACKED, bool DQ>
-__global__ __launch_bounds__(256) void attn32_q_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                       const float* __restrict__ v, const float* __restrict__ d_o,
-                                                       const float* __restrict__ o_in, const float* __restrict__ lse_in,
-                                                       float* __restrict__ dvec, const int32_t* __restrict__ seg_start,
-                                                       float* __restrict__ out, float* __restrict__ lse_out, int B,
-                                                       int Hq, int Hkv, int S, float scale, int causal) {
+// One global -> LDS copy of a wave: 16 (4) bytes per lane from src + voff (lanes past `bytes` get zeros)
+// to dst + 16 lane (4 lane), dst wave-uniform.
+__device__ __forceinline__ void lds_copy16(const float* src, int bytes, char* dst, uint32_t voff) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
+}
+__device__ __forceinline__ void lds_copy4(const float* src, int bytes, char* dst, uint32_t voff) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, voff, 0, 0, 0);
+}
+
+template <int DH>
+struct ALay {
+  static constexpr int kRowB = DH == 64 ? 256 : 512;  // 96: chunks 24-31 of a row stay empty (zeros)
+  static constexpr int kTile = kPos * kRowB;
+  static constexpr int kSlots = kRowB / 16;           // lanes per row of a 1 KiB copy
+  static constexpr int kM = kTile / 8192;             // copies per wave and tile
+  static constexpr int kC = DH / 16;                  // chunks per lane and row
+  static constexpr int kB = DH / 16;                  // 16-row accumulator blocks over head_dim
+};
+
+// The per-lane constants of a wave.
+template <int DH>
+struct ALane {
   using L = ALay<DH>;
-  __shared__ __attribute__((aligned(16))) float kt[32 * L::kPr];
-  __shared__ __attribute__((aligned(16))) float vt[32 * (DQ ? L::kPr : L::kPc)];
-  const int nqb = (S + 127) / 128, nbh = B * Hq;
-  const int qb = nqb - 1 - (int)(blockIdx.x / nbh), bh = blockIdx.x % nbh;
-  const int b = bh / Hq, head = bh % Hq, kvh = head / (Hq / Hkv);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5;
-  const int qw0 = qb * 128 + 32 * w, qi = qw0 + (lane & 31);
-  const bool qvalid = qi < S;
-  const long qrow = (long)bh * S;
+  int col, g;
+  int rb, rt;            // row-read byte offsets: chunks 0-15 (rb) and, head_dim 96, 16-23 (rt), row `col`
+  int cb, ct;            // column-read byte offsets of row 4 g at s = 0
+  uint32_t src[L::kM];   // global byte offsets of this lane's copies, from the tile's first row
+  __device__ __forceinline__ void init() {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    col = lane & 15;
+    g = lane >> 4;
+    rb = col * L::kRowB + (((8 * (g >> 1) + (g & 1)) ^ col) << 4);
+    rt = col * L::kRowB + (((4 * (g >> 1) + (g & 1)) ^ col) << 4) + 256;
+    cb = 4 * g * L::kRowB + ((col ^ (4 * g)) << 4);
+    ct = 4 * g * L::kRowB + (((col >> 1) ^ (4 * g)) << 4) + 8 * (col & 1) + 256;
+#pragma unroll
+    for (int m = 0; m < L::kM; ++m) {
+      const int row = (64 / L::kSlots) * (w + 8 * m) + lane / L::kSlots;
+      const int c = (lane % L::kSlots) ^ (row & 15);
+      src[m] = 16 * c < 4 * DH ? (uint32_t)(row * 4 * DH + 16 * c) : 0x7ffffff0u;  // past the range: zeros
+    }
+  }
+  // Byte offset within a global row of the lane's chunk c.
+  __device__ __forceinline__ int row_chunk(int c) const {
+    if (DH == 96 && c >= 4) return 16 * (16 + 4 * (g >> 1) + 2 * (c - 4) + (g & 1));
+    return 16 * (16 * (c >> 2) + 8 * (g >> 1) + 2 * (c & 3) + (g & 1));
+  }
+  // Chunk c of tile row 16 half + col.
+  __device__ __forceinline__ f32x4 row(const char* tile, int half, int c) const {
+    const int off = (DH == 96 && c >= 4) ? (rt ^ ((c - 4) << 5)) : (rb ^ ((c & 3) << 5)) + ((c >> 2) << 8);
+    return *reinterpret_cast<const f32x4*>(tile + off + 16 * half * L::kRowB);
+  }
+  // Four head_dims 64 b + 4 col + j (j < 4) of tile row 16 half + 4 g + s.
+  __device__ __forceinline__ f32x4 cols(const char* tile, int half, int s, int b) const {
+    return *reinterpret_cast<const f32x4*>(tile + (cb ^ (s << 4)) + (16 * half + s) * L::kRowB + (b << 8));
+  }
+  // head_dim 96: the last 32, 64 + 2 col + j (j < 2).
+  __device__ __forceinline__ f32x2 cols_tail(const char* tile, int half, int s) const {
+    return *reinterpret_cast<const f32x2*>(tile + (ct ^ (s << 4)) + (16 * half + s) * L::kRowB);
+  }
+  // This wave's copies of the 32 rows from position p0 of a [S][DH] matrix (rows past S as zeros;
+  // nothing read, zeros written, when not live).
+  __device__ __forceinline__ void copy(const float* m, int p0, int S, char* tile, bool live) const {
+    const int rows = S - p0 < kPos ? S - p0 : kPos;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int i = 0; i < L::kM; ++i)
+      lds_copy16(m + (live ? (long)p0 * DH : 0), live ? rows * 4 * DH : 0, tile + 1024 * (w + 8 * i), src[i]);
+  }
+  // The lane's chunks of a global row as the B operand of the head_dim products.
+  __device__ __forceinline__ void load_row(const float* row, bool valid, f32x4 (&x)[L::kC]) const {
+#pragma unroll
+    for (int c = 0; c < L::kC; ++c) {
+      x[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (valid) x[c] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(row) + row_chunk(c));
+    }
+  }
+  // acc[half] = tile rows . x (head_dim contraction), the two 16-row chains interleaved.
+  __device__ __forceinline__ void dot_rows(const char* tile, const f32x4 (&x)[L::kC], f32x4 (&acc)[2]) const {
+    acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < L::kC; ++c) {
+      const f32x4 a = row(tile, 0, c), b = row(tile, 1, c);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        acc[0] = mfma4(a[s], x[c][s], acc[0]);
+        acc[1] = mfma4(b[s], x[c][s], acc[1]);
+      }
+    }
+  }
+  // out += tile^T . p over the tile's 32 rows, p[half][r] the weight of row 16 half + 4 g + r.
+  __device__ __forceinline__ void dot_cols(const char* tile, const f32x4 (&p)[2], f32x4 (&out)[L::kB]) const {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int b = 0; b < DH / 64; ++b) {
+          const f32x4 a = cols(tile, half, s, b);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) out[4 * b + j] = mfma4(a[j], p[half][s], out[4 * b + j]);
+        }
+        if constexpr (DH == 96) {
+          const f32x2 a = cols_tail(tile, half, s);
+          out[4] = mfma4(a[0], p[half][s], out[4]);
+          out[5] = mfma4(a[1], p[half][s], out[5]);
+        }
+      }
+  }
+  // Writes acc (head_dim x this lane's position) * mul to the position's global row.
+  __device__ __forceinline__ void store_row(float* row, const f32x4 (&acc)[L::kB], float mul) const {
+#pragma unroll
+    for (int b = 0; b < DH / 64; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<f32x4*>(row + 64 * b + 16 * g + 4 * r) =
+            f32x4{acc[4 * b][r] * mul, acc[4 * b + 1][r] * mul, acc[4 * b + 2][r] * mul, acc[4 * b + 3][r] * mul};
+    if constexpr (DH == 96) {
+#pragma unroll
+      for (int r = 0; r < 4; r += 2)
+        *reinterpret_cast<f32x4*>(row + 64 + 8 * g + 2 * r) =
+            f32x4{acc[4][r] * mul, acc[5][r] * mul, acc[4][r + 1] * mul, acc[5][r + 1] * mul};
+    }
+  }
+};
+// Sum and maximum over the four lanes (g = 0..3) of a column.
+__device__ __forceinline__ float col_sum(float x) {
+  x += __shfl_xor(x, 16, 64);
+  return x + __shfl_xor(x, 32, 64);
+}
+__device__ __forceinline__ float col_max(float x) {
+  x = fmaxf(x, __shfl_xor(x, 16, 64));
+  return fmaxf(x, __shfl_xor(x, 32, 64));
+}
+// The two position blocks of pair p out of n: mirrored (the causal mask: equal work per pair) or
+// adjacent. The second may be n (none).
+__host__ __device__ __forceinline__ void pair_blocks(int p, int n, bool mirror, int& a, int& b) {
+  a = mirror ? p : 2 * p;
+  b = mirror ? n - 1 - p : 2 * p + 1;
+  if (b <= a) b = n;
+}
+__host__ __device__ __forceinline__ int q_heads32(int G) { return G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1; }
+
+// Forward (DQ = false) and dQ (DQ = true). A half-workgroup holds q_heads32(G) heads of one GQA group x
+// 16 (4 / heads) queries: every K/V tile feeds all of them.
+template <int DH, bool PACKED, bool DQ>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DQ ? 2 : 4)))
+void attn32_q_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                     const float* __restrict__ d_o, const float* __restrict__ o_in, const float* __restrict__ lse_in,
+                     float* __restrict__ dvec, const int32_t* __restrict__ seg_start, float* __restrict__ out,
+                     float* __restrict__ lse_out, int B, int Hq, int Hkv, int S, float scale, int causal) {
+  using L = ALay<DH>;
+  __shared__ __attribute__((aligned(1024))) char lds0[2 * L::kTile];  // K, V
+  __shared__ __attribute__((aligned(1024))) char lds1[2 * L::kTile];
+  const int G = Hq / Hkv, hpw = q_heads32(G), R = 16 * (4 / hpw);
+  const int nqb = (S + R - 1) / R, hgb = Hq / hpw, nhg = B * hgb;
+  const int hg = blockIdx.x % nhg, b = hg / hgb, h0 = (hg % hgb) * hpw, kvh = h0 / G;
+  int pa, pb;
+  pair_blocks((int)(blockIdx.x / nhg), nqb, causal && !PACKED, pa, pb);
+  ALane<DH> ln;
+  ln.init();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = w & 3;
+  const int blk = w < 4 ? pa : pb;
+  const int head = h0 + u % hpw, qw0 = blk * R + 16 * (u / hpw), qi = qw0 + ln.col;
+  const bool wave_has = blk < nqb && qw0 < S, qvalid = wave_has && qi < S;
+  const int wq_last = qw0 + 15 < S ? qw0 + 15 : S - 1;
+  const long qrow = (long)(b * Hq + head) * S;
   const float* kh = k + (long)(b * Hkv + kvh) * S * DH;
   const float* vh = v + (long)(b * Hkv + kvh) * S * DH;
   const int32_t* sst = PACKED ? seg_start + (long)b * S : nullptr;
   const float scale_log2 = scale * kLog2e;
 
-  float qx[DH / 2], dx[DQ ? DH / 2 : 1];
-  row_regs<DH>(q + (qrow + qi) * DH, qvalid, qx);
+  f32x4 qx[L::kC], dx[DQ ? L::kC : 1];
+  ln.load_row(q + (qrow + qi) * DH, qvalid, qx);
   float l2q = 0.f, dq_row = 0.f;
   if constexpr (DQ) {
-    row_regs<DH>(d_o + (qrow + qi) * DH, qvalid, dx);
-    float ox[DH / 2];
-    row_regs<DH>(o_in + (qrow + qi) * DH, qvalid, ox);
+    ln.load_row(d_o + (qrow + qi) * DH, qvalid, dx);
+    f32x4 ox[L::kC];
+    ln.load_row(o_in + (qrow + qi) * DH, qvalid, ox);
     float dp = 0.f;
 #pragma unroll
-    for (int e = 0; e < DH / 2; ++e) dp = __builtin_fmaf(dx[e], ox[e], dp);
-    dq_row = dp + __shfl_xor(dp, 32, 64);
-    if (qvalid && h == 0) dvec[qrow + qi] = dq_row;
+    for (int c = 0; c < L::kC; ++c)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) dp = __builtin_fmaf(dx[c][s], ox[c][s], dp);
+    dq_row = col_sum(dp);
+    if (qvalid && ln.g == 0) dvec[qrow + qi] = dq_row;
     l2q = qvalid ? lse_in[qrow + qi] * kLog2e : 0.f;
   }
-  const int wg_q0 = qb * 128;
-  const int wq_last = (qw0 + 31 < S) ? qw0 + 31 : S - 1;
-  const int kv_end = (causal && wg_q0 + 128 < S) ? wg_q0 + 128 : S;
-  const int kv_begin = PACKED ? (sst[wg_q0] / 32) * 32 : 0;
+  // Keys of the workgroup: those of its last block (the latest queries) and, packed, from its first
+  // block's first segment on (adjacent blocks: one contiguous range).
+  const int last = pb < nqb ? pb : pa;
+  const int kv_end = (causal && (last + 1) * R < S) ? (last + 1) * R : S;
+  const int kv_begin = PACKED ? (sst[pa * R] / kPos) * kPos : 0;
+  const int ntiles = (kv_end - kv_begin + kPos - 1) / kPos;
   const int my_sst = (PACKED && qvalid) ? sst[qi] : 0;
-  const int w_sst_first = (PACKED && qw0 < S) ? sst[qw0] : 0;
+  const int w_sst_first = (PACKED && wave_has) ? __builtin_amdgcn_readfirstlane(sst[qw0]) : 0;
+  const int w_sst_last = (PACKED && wave_has) ? __builtin_amdgcn_readfirstlane(sst[wq_last]) : 0;
 
   float m = kNegInf, l = 0.f;
-  f32x16 acc[DH / 32];
+  f32x4 acc[L::kB];
 #pragma unroll
-  for (int db = 0; db < DH / 32; ++db) zero(acc[db]);
-  for (int kv0 = kv_begin; kv0 < kv_end; kv0 += 32) {
-    __syncthreads();
-    tile_in<DH, L::kPr>(kh, kv0, S, kt);
-    tile_in<DH, DQ ? L::kPr : L::kPc>(vh, kv0, S, vt);
-    __syncthreads();
-    if (qw0 >= S || (causal && kv0 > wq_last) || (PACKED && kv0 + 31 < w_sst_first)) continue;
-    f32x16 sacc;
-    zero(sacc);
-    dot_rows<DH, L::kPr>(kt, qx, sacc);  // S^T = K Q^T (keys x this lane's query)
-    // visibility of key kv0 + rrow(r, h) to this lane's query
-    auto visible = [&](int r) {
-      const int kj = kv0 + rrow(r, h);
-      bool ok = qvalid && kj < S && (!causal || kj <= qi);
-      if (PACKED) ok = ok && kj >= my_sst;
-      return ok;
-    };
-    if constexpr (DQ) {
-      f32x16 pacc;
-      zero(pacc);
-      dot_rows<DH, L::kPr>(vt, dx, pacc);  // dP^T = V dO^T
-      f32x16 ds;
+  for (int i = 0; i < L::kB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  ln.copy(kh, kv_begin, S, lds0, true);
+  ln.copy(vh, kv_begin, S, lds0 + L::kTile, true);
+  copies_landed();
+  // The row loads are complete here: tell the compiler, which would wait for them (and for the copies
+  // in flight) at their first use.
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = visible(r) ? fast_exp2(__builtin_fmaf(sacc[r], scale_log2, -l2q)) : 0.f;
-        ds[r] = p * (pacc[r] - dq_row);
-      }
-      dot_cols<DH, L::kPr>(kt, ds, acc);  // dQ^T += K^T dS^T
-    } else {
-      float mx = kNegInf;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        sacc[r] = visible(r) ? sacc[r] * scale_log2 : kNegInf;
-        mx = fmaxf(mx, sacc[r]);
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mn = fmaxf(m, mx);
-      const float base = (mn == kNegInf) ? 0.f : mn;
-      const float alpha = fast_exp2(m - base);  // m = -inf: 0 (O and l are 0)
-      l *= alpha;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        sacc[r] = fast_exp2(sacc[r] - base);
-        l += sacc[r];
-      }
-      m = mn;
-#pragma unroll
-      for (int db = 0; db < DH / 32; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
-      dot_cols<DH, L::kPc>(vt, sacc, acc);  // O^T += V^T P^T
-    }
+  for (int c = 0; c < L::kC; ++c) {
+    asm volatile("" : "+v"(qx[c]));
+    if constexpr (DQ) asm volatile("" : "+v"(dx[c]));
   }
-  if (!qvalid) return;
+
+  auto body = [&](int t, const char* cur, char* nxt) __attribute__((always_inline)) {
+    const int kv0 = kv_begin + t * kPos;
+    ln.copy(kh, kv0 + kPos, S, nxt, t + 1 < ntiles);
+    ln.copy(vh, kv0 + kPos, S, nxt + L::kTile, t + 1 < ntiles);
+    if (wave_has && !(causal && kv0 > wq_last) && !(PACKED && kv0 + kPos - 1 < w_sst_first)) {
+      f32x4 sc[2];
+      ln.dot_rows(cur, qx, sc);  // S^T = K Q^T
+      // Only tiles across the wave's diagonal, the sequence end or a segment start hold hidden pairs.
+      const bool need_mask = (causal && kv0 + kPos - 1 > qw0) || kv0 + kPos > S || (PACKED && kv0 < w_sst_last);
+      const int hi = (causal ? (qi < S - 1 ? qi : S - 1) : S - 1) - kv0 - 4 * ln.g, lo = my_sst - kv0 - 4 * ln.g;
+      auto visible = [&](int half, int r) { return 16 * half + r <= hi && (!PACKED || 16 * half + r >= lo); };
+      if constexpr (DQ) {
+        f32x4 dp[2];
+        ln.dot_rows(cur + L::kTile, dx, dp);  // dP^T = V dO^T
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[half][r] = fast_exp2(__builtin_fmaf(sc[half][r], scale_log2, -l2q));
+        if (need_mask) {
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[half][r] = visible(half, r) ? sc[half][r] : 0.f;
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[half][r] *= dp[half][r] - dq_row;
+        ln.dot_cols(cur, sc, acc);  // dQ^T += K^T dS^T
+      } else {
+        float mx = kNegInf;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[half][r] *= scale_log2;
+        if (need_mask) {
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[half][r] = visible(half, r) ? sc[half][r] : kNegInf;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fmaxf(sc[0][r], sc[1][r]));
+        const float mn = fmaxf(m, col_max(mx));
+        const float base = (mn == kNegInf) ? 0.f : mn;
+        // O and l are rescaled when some query's maximum rose; alpha is 1 for the others.
+        if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
+          const float alpha = fast_exp2(m - base);  // m = -inf: 0 (O and l are 0)
+          l *= alpha;
+#pragma unroll
+          for (int i = 0; i < L::kB; ++i) acc[i] *= alpha;
+          m = mn;
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            sc[half][r] = fast_exp2(sc[half][r] - base);
+            l += sc[half][r];
+          }
+        ln.dot_cols(cur + L::kTile, sc, acc);  // O^T += V^T P^T
+      }
+    }
+    copies_landed();
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    body(t, lds0, lds1);
+    if (t + 1 < ntiles) body(t + 1, lds1, lds0);
+  }
   if constexpr (DQ) {
-    store_rows<DH>(out + (qrow + qi) * DH, acc, scale);
+    if (qvalid) ln.store_row(out + (qrow + qi) * DH, acc, scale);
   } else {
-    const float lt = l + __shfl_xor(l, 32, 64);
-    if (h == 0) lse_out[qrow + qi] = (lt > 0.f) ? (m + fast_log2(lt)) * kLn2 : kNegInf;
-    store_rows<DH>(out + (qrow + qi) * DH, acc, lt > 0.f ? 1.f / lt : 0.f);
+    const float lt = col_sum(l);
+    if (!qvalid) return;
+    if (ln.g == 0) lse_out[qrow + qi] = (lt > 0.f) ? (m + fast_log2(lt)) * kLn2 : kNegInf;
+    ln.store_row(out + (qrow + qi) * DH, acc, lt > 0.f ? 1.f / lt : 0.f);
   }
 }
 
-// dK, dV: 128 keys of one kv head per workgroup (key block 0 first), each wave 32 keys holding its
-// K and V rows in registers; items (query head of the group, 32-query tile) visit the queries
-// that see the block; dK^T and dV^T accumulate in registers (no atomics).
+// dK, dV: a half-workgroup holds a block of 64 keys of one kv head, each wave 16 of them with their K
+// and V rows; items (query head h of the group, 32-query tile t) visit the queries that see the pair of
+// blocks. They are dealt to nsplit workgroups, item (h, t) to (h + t) % nsplit (attn32_dkv_splits), so
+// that a key's partial sums do not depend on the block it is paired with (one packed segment gives the
+// causal result bit for bit); with several, each writes an fp32 partial
+// part[split][dK | dV][b][kv head][key][d], which attn32_dkv_reduce_kernel sums in split order.
 template <int DH, bool PACKED>
-__global__ __launch_bounds__(256) void attn32_dkv_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                         const float* __restrict__ v, const float* __restrict__ d_o,
-                                                         const float* __restrict__ lse, const float* __restrict__ dvec,
-                                                         const int32_t* __restrict__ seg_start, float* __restrict__ dk,
-                                                         float* __restrict__ dv, int B, int Hq, int Hkv, int S, float scale,
-                                                         int causal) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+void attn32_dkv_kernel(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+                       const float* __restrict__ d_o, const float* __restrict__ lse, const float* __restrict__ dvec,
+                       const int32_t* __restrict__ seg_start, float* __restrict__ dk, float* __restrict__ dv, int B,
+                       int Hq, int Hkv, int S, float scale, int causal, int nsplit, float* __restrict__ part) {
   using L = ALay<DH>;
-  __shared__ __attribute__((aligned(16))) float qt[32 * L::kPr];
-  __shared__ __attribute__((aligned(16))) float ot[32 * L::kPr];
-  __shared__ float lt[32], dt[32];
-  const int nbh = B * Hkv;
-  const int kb = blockIdx.x / nbh, bh = blockIdx.x % nbh;
-  const int b = bh / Hkv, kvh = bh % Hkv, G = Hq / Hkv;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5;
-  const int k0 = kb * 128, kw0 = k0 + 32 * w, kj = kw0 + (lane & 31);
-  const bool kvalid = kj < S;
+  __shared__ __attribute__((aligned(1024))) char lds0[2 * L::kTile + 512];  // Q, dO, L (32 of 64), D (32 of 64)
+  __shared__ __attribute__((aligned(1024))) char lds1[2 * L::kTile + 512];
+  const int G = Hq / Hkv, nkb = (S + 63) / 64, nbh = B * Hkv;
+  const int split = blockIdx.x % nsplit, bh = (blockIdx.x / nsplit) % nbh, b = bh / Hkv, kvh = bh % Hkv;
+  int ba, bb;
+  pair_blocks((int)(blockIdx.x / nsplit / nbh), nkb, causal && !PACKED, ba, bb);
+  ALane<DH> ln;
+  ln.init();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blk = w < 4 ? ba : bb, kw0 = blk * 64 + 16 * (w & 3), kj = kw0 + ln.col;
+  const bool wave_has = blk < nkb && kw0 < S, kvalid = wave_has && kj < S;
   const long krow = (long)bh * S;
   const float scale_log2 = scale * kLog2e;
   const int32_t* sst = PACKED ? seg_start + (long)b * S : nullptr;
 
-  float kx[DH / 2], vx[DH / 2];
-  row_regs<DH>(k + (krow + kj) * DH, kvalid, kx);
-  row_regs<DH>(v + (krow + kj) * DH, kvalid, vx);
-  const int q_begin = causal ? (k0 / 32) * 32 : 0;
-  int q_end = S, my_lim = S;
+  f32x4 kx[L::kC], vx[L::kC];
+  ln.load_row(k + (krow + kj) * DH, kvalid, kx);
+  ln.load_row(v + (krow + kj) * DH, kvalid, vx);
+  // Query tiles [t0, t1) see the workgroup's keys; queries q < my_lim see key kj (packed: those of its
+  // segment), and the wave's keys none from w_end on.
+  const int t0 = causal ? ba * (64 / kPos) : 0;
+  int t1 = (S + kPos - 1) / kPos, my_lim = S, w_lim = S, w_end = S;
   if (PACKED) {
-    const int klast = (k0 + 127 < S) ? k0 + 127 : S - 1;
-    int lo = 0, hi = S;  // first position whose segment starts after klast
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (sst[mid] > klast) hi = mid;
-      else lo = mid + 1;
-    }
-    q_end = lo;
-    if (kvalid) {  // the end of key kj's segment
-      lo = kj;
-      hi = q_end;
+    auto above = [&](int x) {  // the end of position x's segment
+      int lo = x, hi = S;
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (sst[mid] > kj) hi = mid;
+        if (sst[mid] > x) hi = mid;
         else lo = mid + 1;
       }
-      my_lim = lo;
+      return lo;
+    };
+    const int last = bb < nkb ? bb : ba, wl = kw0 + 15 < S ? kw0 + 15 : S - 1;
+    t1 = (__builtin_amdgcn_readfirstlane(above(last * 64 + 63 < S ? last * 64 + 63 : S - 1)) + kPos - 1) / kPos;
+    if (kvalid) my_lim = above(kj);
+    w_lim = __builtin_amdgcn_readfirstlane(my_lim);  // the first key's: the smallest
+    if (wave_has) w_end = __builtin_amdgcn_readfirstlane(above(wl));
+  }
+  struct Item {
+    int h, t;
+  };
+  auto settle = [&](Item x) __attribute__((always_inline)) {  // the first item of this split from x on (h = G: none)
+    while (x.h < G && x.t >= t1) {
+      ++x.h;
+      int r = (split - x.h - t0) % nsplit;
+      if (r < 0) r += nsplit;
+      x.t = t0 + r;
     }
-  }
-  f32x16 dka[DH / 32], dva[DH / 32];
+    return x;
+  };
+
+  f32x4 dka[L::kB], dva[L::kB];
 #pragma unroll
-  for (int db = 0; db < DH / 32; ++db) {
-    zero(dka[db]);
-    zero(dva[db]);
-  }
-  for (int hh = 0; hh < G; ++hh) {
-    const long qrow = (long)(b * Hq + kvh * G + hh) * S;
-    for (int q0 = q_begin; q0 < q_end; q0 += 32) {
-      __syncthreads();
-      tile_in<DH, L::kPr>(q + qrow * DH, q0, S, qt);
-      tile_in<DH, L::kPr>(d_o + qrow * DH, q0, S, ot);
-      if (threadIdx.x < 32) {
-        const int qq = q0 + threadIdx.x;
-        lt[threadIdx.x] = qq < S ? lse[qrow + qq] * kLog2e : 0.f;
-        dt[threadIdx.x] = qq < S ? dvec[qrow + qq] : 0.f;
-      }
-      __syncthreads();
-      if (kw0 >= S) continue;                 // the wave holds no key
-      if (causal && q0 + 31 < kw0) continue;  // every query of the tile precedes the wave's keys
-      f32x16 sacc, pacc;
-      zero(sacc);
-      zero(pacc);
-      dot_rows<DH, L::kPr>(qt, kx, sacc);  // S = Q K^T (queries x this lane's key)
-      dot_rows<DH, L::kPr>(ot, vx, pacc);  // dP = dO V^T
-      f32x16 p, ds;
+  for (int i = 0; i < L::kB; ++i) dka[i] = dva[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Copies of an item into a stage: Q and dO rows, L and D (waves 0 and 1, 32 floats each).
+  auto copy = [&](Item x, char* st) __attribute__((always_inline)) {
+    const bool live = x.h < G;
+    const int q0 = x.t * kPos;
+    const long qrow = (long)(b * Hq + kvh * G + (live ? x.h : 0)) * S;
+    ln.copy(q + qrow * DH, q0, S, st, live);
+    ln.copy(d_o + qrow * DH, q0, S, st + L::kTile, live);
+    if (w < 2) {
+      const int rows = S - q0 < kPos ? S - q0 : kPos;
+      lds_copy4((w ? dvec : lse) + qrow + (live ? q0 : 0), live ? rows * 4 : 0, st + 2 * L::kTile + 256 * w,
+                  4u * (threadIdx.x & 63));
+    }
+  };
+  auto body = [&](Item x, Item next, const char* cur, char* nxt) __attribute__((always_inline)) {
+    copy(next, nxt);
+    const int q0 = x.t * kPos;
+    if (wave_has && !(causal && q0 + kPos - 1 < kw0) && !(PACKED && q0 >= w_end)) {
+      f32x4 p[2], ds[2];
+      ln.dot_rows(cur, kx, p);              // S = Q K^T (queries x this lane's key)
+      ln.dot_rows(cur + L::kTile, vx, ds);  // dP = dO V^T
+      const float* sl = reinterpret_cast<const float*>(cur + 2 * L::kTile);
+      const bool need_mask = (causal && q0 < kw0 + 15) || q0 + kPos > S || (PACKED && q0 + kPos > w_lim);
+      const int lo = causal ? kj - q0 - 4 * ln.g : -kPos, hi = my_lim - q0 - 4 * ln.g;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qq = q0 + rrow(r, h);
-        const bool ok = kvalid && qq < S && (!causal || kj <= qq) && qq < my_lim;
-        p[r] = ok ? fast_exp2(__builtin_fmaf(sacc[r], scale_log2, -lt[rrow(r, h)])) : 0.f;
-        ds[r] = p[r] * (pacc[r] - dt[rrow(r, h)]);
+      for (int half = 0; half < 2; ++half) {
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(sl + 16 * half + 4 * ln.g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[half][r] = fast_exp2(__builtin_fmaf(p[half][r], scale_log2, -l4[r] * kLog2e));
       }
-      dot_cols<DH, L::kPr>(ot, p, dva);   // dV^T += dO^T P
-      dot_cols<DH, L::kPr>(qt, ds, dka);  // dK^T += Q^T dS
+      if (need_mask) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) p[half][r] = (16 * half + r >= lo && 16 * half + r < hi) ? p[half][r] : 0.f;
+      }
+      ln.dot_cols(cur + L::kTile, p, dva);  // dV^T += dO^T P
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(sl + 64 + 16 * half + 4 * ln.g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ds[half][r] = p[half][r] * (ds[half][r] - d4[r]);
+      }
+      ln.dot_cols(cur, ds, dka);  // dK^T += Q^T dS
+    }
+    copies_landed();
+  };
+  Item x = settle(Item{-1, t1});
+  if (x.h < G) {
+    copy(x, lds0);
+    copies_landed();
+#pragma unroll
+    for (int c = 0; c < L::kC; ++c) asm volatile("" : "+v"(kx[c]), "+v"(vx[c]));
+    while (true) {
+      const Item y = settle(Item{x.h, x.t + nsplit});
+      body(x, y, lds0, lds1);
+      if (y.h >= G) break;
+      x = settle(Item{y.h, y.t + nsplit});
+      body(y, x, lds1, lds0);
+      if (x.h >= G) break;
     }
   }
   if (!kvalid) return;
-  store_rows<DH>(dk + (krow + kj) * DH, dka, scale);
-  store_rows<DH>(dv + (krow + kj) * DH, dva, 1.f);
+  const long plane = (long)nbh * S * DH;
+  if (nsplit > 1) {
+    dk = part + 2L * split * plane;
+    dv = dk + plane;
+  }
+  ln.store_row(dk + (krow + kj) * DH, dka, scale);
+  ln.store_row(dv + (krow + kj) * DH, dva, 1.f);
+}
+
+// dK (blockIdx.y 0) or dV (1) = the sum of the nsplit partials in split order. plane: floats, a multiple of 4.
+__global__ __launch_bounds__(256) void attn32_dkv_reduce_kernel(const float* __restrict__ part, int nsplit, long plane,
+                                                                float* __restrict__ dk, float* __restrict__ dv) {
+  const long e = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (e >= plane) return;
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+  for (int sp = 0; sp < nsplit; ++sp) x += *reinterpret_cast<const f32x4*>(part + (2L * sp + blockIdx.y) * plane + e);
+  *reinterpret_cast<f32x4*>((blockIdx.y ? dv : dk) + e) = x;
 }
 
 }  // namespace f32k
@@ -815,11 +1013,33 @@ hipError_t launch_lce32_bwd(const LceHead32& h, const float* H, const int64_t* t
   return hipSuccess;
 }
 
+// Splits of each pair of key blocks in the fp32 dK/dV pass. One 8-wave workgroup per CU: the count that
+// takes the fewest rounds x items (an item, 32 queries of one head against a pair: about 7 us) plus
+// the partials' write and read (28 MB in the time of an item).
+int attn32_dkv_splits(int b, int hq, int hkv, int s, int dh) {
+  if (b < 1 || hkv < 1 || s < 1 || hq % hkv) return 1;
+  const long pairs = ((s + 63) / 64 + 1) / 2, wgs = pairs * b * hkv, items = (long)(hq / hkv) * ((s + kPos - 1) / kPos);
+  const long plane = (long)b * hkv * s * dh * 4;
+  auto cost = [&](long ns) { return (wgs * ns + kNumCU - 1) / kNumCU * ((items + ns - 1) / ns) * 28000000L + (ns > 1 ? 4 * ns * plane : 0); };
+  int best = 1;
+  for (int ns = 2; ns <= 16 && ns <= items; ++ns)
+    if (cost(ns) < cost(best)) best = ns;
+  return best;
+}
+// D, then, from the next 256-byte boundary, the partials of a split dK/dV pass.
+size_t attn32_bwd_workspace(int b, int hq, int hkv, int s, int dh, int ns) {
+  return (size_t)b * hq * s * sizeof(float) + (ns > 1 ? 256 + (size_t)ns * 2 * b * hkv * s * dh * sizeof(float) : 0);
+}
+
 namespace {
+dim3 grid32_q(const AttnShape& sh) {
+  const int hpw = q_heads32(sh.hq / sh.hkv), R = 16 * (4 / hpw);
+  return dim3(((sh.s + R - 1) / R + 1) / 2 * sh.b * (sh.hq / hpw));
+}
 template <int DH>
 hipError_t fwd32_dh(const AttnShape& sh, const float* q, const float* k, const float* v, const int32_t* sst, float* o,
                     float* lse, hipStream_t st) {
-  dim3 grid(((sh.s + 127) / 128) * sh.b * sh.hq), block(256);
+  const dim3 grid = grid32_q(sh), block(512);
   if (sst) hipLaunchKernelGGL((attn32_q_kernel<DH, true, false>), grid, block, 0, st, q, k, v, nullptr, nullptr, nullptr, nullptr, sst, o, lse, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
   else hipLaunchKernelGGL((attn32_q_kernel<DH, false, false>), grid, block, 0, st, q, k, v, nullptr, nullptr, nullptr, nullptr, sst, o, lse, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
   return hipGetLastError();
@@ -827,15 +1047,20 @@ hipError_t fwd32_dh(const AttnShape& sh, const float* q, const float* k, const f
 template <int DH>
 hipError_t bwd32_dh(const AttnShape& sh, const float* q, const float* k, const float* v, const float* o,
                     const float* lse, const float* d_o, const int32_t* sst, float* dq, float* dk, float* dv,
-                    float* dvec, hipStream_t st) {
-  dim3 qgrid(((sh.s + 127) / 128) * sh.b * sh.hq), block(256);
+                    float* dvec, int ns, hipStream_t st) {
+  const dim3 qgrid = grid32_q(sh), block(512);
   if (sst) hipLaunchKernelGGL((attn32_q_kernel<DH, true, true>), qgrid, block, 0, st, q, k, v, d_o, o, lse, dvec, sst, dq, nullptr, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
   else hipLaunchKernelGGL((attn32_q_kernel<DH, false, true>), qgrid, block, 0, st, q, k, v, d_o, o, lse, dvec, sst, dq, nullptr, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  dim3 kgrid(((sh.s + 127) / 128) * sh.b * sh.hkv);
-  if (sst) hipLaunchKernelGGL((attn32_dkv_kernel<DH, true>), kgrid, block, 0, st, q, k, v, d_o, lse, dvec, sst, dk, dv, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
-  else hipLaunchKernelGGL((attn32_dkv_kernel<DH, false>), kgrid, block, 0, st, q, k, v, d_o, lse, dvec, sst, dk, dv, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal);
+  float* part = reinterpret_cast<float*>(((uintptr_t)(dvec + (size_t)sh.b * sh.hq * sh.s) + 255) / 256 * 256);
+  const dim3 kgrid(((sh.s + 63) / 64 + 1) / 2 * sh.b * sh.hkv * ns);
+  if (sst) hipLaunchKernelGGL((attn32_dkv_kernel<DH, true>), kgrid, block, 0, st, q, k, v, d_o, lse, dvec, sst, dk, dv, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal, ns, part);
+  else hipLaunchKernelGGL((attn32_dkv_kernel<DH, false>), kgrid, block, 0, st, q, k, v, d_o, lse, dvec, sst, dk, dv, sh.b, sh.hq, sh.hkv, sh.s, sh.scale, sh.causal, ns, part);
+  e = hipGetLastError();
+  if (e != hipSuccess || ns == 1) return e;
+  const long plane = (long)sh.b * sh.hkv * sh.s * DH;
+  hipLaunchKernelGGL(attn32_dkv_reduce_kernel, dim3((unsigned)((plane / 4 + 255) / 256), 2), dim3(256), 0, st, part, ns, plane, dk, dv);
   return hipGetLastError();
 }
 }  // namespace
@@ -852,11 +1077,11 @@ hipError_t launch_attn32_fwd(const AttnShape& sh, const float* q, const float* k
 
 hipError_t launch_attn32_bwd(const AttnShape& sh, const float* q, const float* k, const float* v, const float* o,
                              const float* lse, const float* d_o, const int32_t* seg_start, float* dq, float* dk,
-                             float* dv, float* dvec, hipStream_t st) {
+                             float* dv, float* dvec, int nsplit, hipStream_t st) {
   switch (sh.dh) {
-    case 64: return bwd32_dh<64>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, st);
-    case 96: return bwd32_dh<96>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, st);
-    case 128: return bwd32_dh<128>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, st);
+    case 64: return bwd32_dh<64>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, nsplit, st);
+    case 96: return bwd32_dh<96>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, nsplit, st);
+    case 128: return bwd32_dh<128>(sh, q, k, v, o, lse, d_o, seg_start, dq, dk, dv, dvec, nsplit, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -99,9 +99,12 @@ hipError_t launch_lce32_bwd(const LceHead32& h, const float* H, const int64_t* t
                             float* dW, float* Gbuf, hipStream_t stream);
 hipError_t launch_attn32_fwd(const AttnShape& sh, const float* q, const float* k, const float* v,
                              const int32_t* seg_start, float* o, float* lse, hipStream_t stream);
-// dvec: fp32 [b][hq][s] (D = rowsum(dO * O), formed by the dQ pass for the dK/dV pass).
+// Splits of the fp32 dK/dV pass (1: none), and the backward's workspace with them: D, then the partials.
+int attn32_dkv_splits(int b, int hq, int hkv, int s, int dh);
+size_t attn32_bwd_workspace(int b, int hq, int hkv, int s, int dh, int nsplit);
+// dvec: the workspace, D = rowsum(dO * O) fp32 [b][hq][s] first (formed by the dQ pass for the dK/dV pass).
 hipError_t launch_attn32_bwd(const AttnShape& sh, const float* q, const float* k, const float* v, const float* o,
                              const float* lse, const float* d_o, const int32_t* seg_start, float* dq, float* dk,
-                             float* dv, float* dvec, hipStream_t stream);
+                             float* dv, float* dvec, int nsplit, hipStream_t stream);
 
 }  // namespace mtp

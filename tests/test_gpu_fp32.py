@@ -190,6 +190,51 @@ def test_attention_fp32_parity(shape, causal):
     _attn_check(_attn32(q, k, v, do, scale, causal=causal), q, k, v, do, scale, causal=causal, tag=str(shape))
 
 
+# Edges of the 16-query and 16-key waves, of the 32-position tiles, of the 64-key blocks and of the pairs of
+# blocks (odd and even counts, one block alone) for workgroups of 4, 2 and 1 heads; the last with enough
+# items for 16 splits of the dK/dV pass.
+@pytest.mark.parametrize("shape", [(1, 4, 1, 15, 64), (1, 2, 1, 16, 96), (1, 3, 3, 17, 128), (2, 6, 2, 31, 64),
+                                   (1, 4, 4, 33, 96), (1, 8, 1, 64, 128), (1, 2, 2, 65, 64), (1, 4, 2, 129, 96),
+                                   (1, 3, 1, 192, 128), (1, 4, 1, 513, 64)])
+@pytest.mark.parametrize("mask", ["causal", "full", "packed"])
+def test_attention_fp32_block_edges(shape, mask):
+    b, hq, hkv, s, d = shape
+    g = torch.Generator().manual_seed(11)
+    q, do = (torch.randn(b, hq, s, d, generator=g) for _ in range(2))
+    k, v = (torch.randn(b, hkv, s, d, generator=g) for _ in range(2))
+    sid = sst = None
+    if mask == "packed":
+        sid, sst = oatt.segments_from_lengths([s // 3, 1, s - 1 - s // 3])
+        sid, sst = sid[None].repeat(b, 1), sst[None].repeat(b, 1)
+    scale = 1 / math.sqrt(d)
+    got = _attn32(q, k, v, do, scale, causal=mask != "full", sid=sid, sst=sst)
+    _attn_check(got, q, k, v, do, scale, causal=mask != "full", sid=sid, tag=f"{shape} {mask}")
+
+
+def test_attention_fp32_workspace_for_d_alone_runs_unsplit():
+    """mtp_attn_bwd_f32 with room for D only gives the split pass's gradients, summed in another order."""
+    from mlx_train_perf import _native
+    from mlx_train_perf.attention.api import kernel_backward, kernel_forward
+
+    b, hq, hkv, s, d = 1, 4, 2, 300, 64
+    lib = _native.load()
+    assert lib.mtp_attn_bwd_f32_workspace_bytes(b, hq, hkv, s, d) > 4 * b * hq * s
+    g = torch.Generator().manual_seed(3)
+    q, do = (torch.randn(b, hq, s, d, generator=g).cuda() for _ in range(2))
+    k, v = (torch.randn(b, hkv, s, d, generator=g).cuda() for _ in range(2))
+    o, lse = kernel_forward(q, k, v, scale=0.125)
+    want = kernel_backward(q, k, v, o, lse, do, scale=0.125)
+    ws = torch.empty(b * hq * s, device="cuda")
+    got = [torch.empty_like(x) for x in (q, k, v)]
+    rc = lib.mtp_attn_bwd_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), do.data_ptr(), b,
+                              hq, hkv, s, d, 0.125, 1, None, None, *(x.data_ptr() for x in got), ws.data_ptr(),
+                              ws.numel() * 4, _native.stream_of(q))
+    assert rc == _native.MTP_OK
+    assert torch.equal(got[0], want[0])
+    for a, w in zip(got[1:], want[1:]):   # sums of at most 600 terms of size ~1 in another order: 600 eps
+        assert float((a - w).abs().max()) < 600 * 2 ** -24 * float(w.abs().max())
+
+
 @pytest.mark.parametrize("lengths", [[5, 7], [1, 60, 3, 200], [257], [40, 1, 1, 88]])
 def test_attention_fp32_packed(lengths):
     """Packed rows (B = 2) against the block-diagonal oracle; one segment equals plain causal
