@@ -189,6 +189,14 @@ def test_trainable_head_dw_parity(n, d, v, chunk):
     assert rel_l2(wd.grad.cpu(), odw) <= 1e-2
 
 
+# Token counts around the 64-deep stages of the dW product and hidden dims around its 256-column tiles,
+# several chunks and a vocabulary that ends inside a tile.
+@pytest.mark.parametrize(("n", "d", "v", "chunk"), [(1, 64, 300, 256), (63, 72, 300, None), (65, 256, 700, 256),
+                                                    (127, 264, 513, None), (257, 200, 300, 256), (447, 320, 300, None)])
+def test_trainable_head_dw_ragged_tokens(n, d, v, chunk):
+    test_trainable_head_dw_parity(n, d, v, chunk)
+
+
 @pytest.mark.parametrize(("v", "d"), [(1027, 192), (300, 64), (5000, 512)])
 def test_head_transpose_exact(v, d):
     """mtp_lce_head_transpose: w_t[:, :v] == w.T bitwise, zero padding up to the row pitch."""
