@@ -197,7 +197,150 @@ __device__ __forceinline__ void gemm128(const SA& sa, const SB& sb, int K, float
   }
 }
 
+// The waves' copies have landed and their LDS reads are done, for the whole workgroup.
+__device__ __forceinline__ void copies_landed() {
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
+}
+// One global -> LDS copy of a wave: 16 (4) bytes per lane from src + voff (lanes past `bytes` get zeros)
+// to dst + 16 lane (4 lane), dst wave-uniform.
+__device__ __forceinline__ void lds_copy16(const float* src, int bytes, char* dst, uint32_t voff) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
+}
+__device__ __forceinline__ void lds_copy4(const float* src, int bytes, char* dst, uint32_t voff) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, voff, 0, 0, 0);
+}
+
+// ------------------------------------------------------------------------------------------
+// The same product on copied tiles (dense operands whose rows are multiples of 16 bytes): 32-deep stages of
+// 16 KiB per operand, copied global -> LDS one stage ahead, one barrier per stage; two workgroups per CU.
+// The matrix pipe bounds it (4096 MFMA cycles per wave and stage against 32 KiB copied and 16 KiB
+// read); the register-staged core above stalls on its loads and LDS writes. N = 1024, D = 512, V = 32000, the
+// kernels' times in one trace: forward 363 -> 305 us, gradient tiles 391 -> 343, dH 367 -> 302; the whole
+// step 1043 -> 827 us (122 of the 153 TFLOP/s a library fp32 matrix product reaches). Two 256-register
+// waves per SIMD: left to a budget of 512 the compiler moved the accumulators between VGPRs and AGPRs
+// in every stage.
+//   RowOp: k along a row: [128 rows][32 k], chunk c (4 k) of row r at slot c ^ swz32(r); a lane reads chunk
+//          2 c + h of its row for the 4 steps of c.
+//   ColOp: k-major: [32 k][128 columns]; a lane reads columns 2 i and 2 i + 1 of the k rows of its half, so
+//          block b of a wave holds the columns 2 i + b.
+// Lane half h contracts k = 8 c + 4 h + s at step s of c, in both. Rows, k and columns past the end read
+// as zeros or (columns of a k-major operand) as neighbours whose results are not stored.
+// ------------------------------------------------------------------------------------------
+constexpr int kDK = 32, kOpB = 16384;
+__device__ __forceinline__ int swz32(int r) { return (r ^ ((r >> 3) & 3)) & 7; }
+__device__ __forceinline__ int range31(long bytes) { return bytes <= 0 ? 0 : bytes > 0x7fffffffL ? 0x7fffffff : (int)bytes; }
+
+struct RowOp {
+  const float* p;  // tile row 0, k = 0
+  long ld;
+  int rows, K;     // rows from the tile start, contraction length
+  uint32_t voff;   // this lane's offset in its wave's copy 0; copy m lies 32 m rows on
+  int ck;          // first k of the lane's chunk
+  __device__ __forceinline__ RowOp(const float* p_, long ld_, int rows_, int K_) : p(p_), ld(ld_), rows(rows_ < kT ? rows_ : kT), K(K_) {
+    const int lane = threadIdx.x & 63, row = 8 * (threadIdx.x >> 6) + (lane >> 3);
+    ck = 4 * ((lane & 7) ^ swz32(row));
+    voff = 4u * (uint32_t)(row * (int)ld + ck);
+  }
+  static __device__ __forceinline__ int pos(int b, int i) { return 32 * b + i; }
+  __device__ __forceinline__ void copy(int kt, char* dst) const {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), left = K - kt * kDK;
+    // (a gradient tile's row may end inside a chunk: its zeros up to the chunk's end are read too)
+    const int bytes = left > 0 ? range31(4 * ((rows - 1) * ld + ((left + 3) & ~3))) : 0;
+    const uint32_t v = ck < left ? voff : 0x60000000u;  // past the end of its row: nothing
+#pragma unroll
+    for (int m = 0; m < 4; ++m) lds_copy16(p + kt * kDK, bytes, dst + 1024 * (4 * m + w), v + 128u * m * (uint32_t)ld);
+  }
+  __device__ __forceinline__ void frags(const char* st, int first, int c, float (&v)[2][4]) const {
+    const int i = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1, row = first + i;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(st + row * 128 + (((h ^ swz32(row)) << 4) ^ (c << 5)) + 4096 * b);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) v[b][s] = x[s];
+    }
+  }
+};
+struct ColOp {
+  const float* p;  // k = 0, tile column 0
+  long ld;
+  int cols, K;     // columns from the tile start to the end of the row, contraction length
+  uint32_t voff;   // this lane's offset in its wave's copy 0; copy m lies 8 m k rows on
+  __device__ __forceinline__ ColOp(const float* p_, long ld_, int cols_, int K_) : p(p_), ld(ld_), cols(cols_), K(K_) {
+    const int lane = threadIdx.x & 63;
+    voff = 4u * (uint32_t)((2 * (threadIdx.x >> 6) + (lane >> 5)) * (int)ld + 4 * (lane & 31));
+  }
+  static __device__ __forceinline__ int pos(int b, int i) { return 2 * i + b; }
+  __device__ __forceinline__ void copy(int kt, char* dst) const {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), left = K - kt * kDK;
+    const int bytes = left > 0 ? range31(4 * ((left - 1) * ld + cols)) : 0;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) lds_copy16(p + kt * kDK * ld, bytes, dst + 1024 * (4 * m + w), voff + 32u * m * (uint32_t)ld);
+  }
+  __device__ __forceinline__ void frags(const char* st, int first, int c, float (&v)[2][4]) const {
+    const int i = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const f32x2 x = *reinterpret_cast<const f32x2*>(st + (8 * c + 4 * h + s) * 512 + 4 * (first + 2 * i));
+      v[0][s] = x[0];
+      v[1][s] = x[1];
+    }
+  }
+};
+// acc[bi][bj] = C[64 (w & 1) + OA::pos(bi, ..)][64 (w >> 1) + OB::pos(bj, ..)]; s0 and s1 hold A, then B.
+template <class OA, class OB>
+__device__ __forceinline__ void gemm128_copied(const OA& oa, const OB& ob, int K, char* s0, char* s1, f32x16 (&acc)[2][2]) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ra = 64 * (w & 1), rb = 64 * (w >> 1);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) zero(acc[i][j]);
+  const int nk = (K + kDK - 1) / kDK;
+  auto stage = [&](int kt, const char* cur, char* nxt) __attribute__((always_inline)) {
+    oa.copy(kt + 1, nxt);  // past the end: nothing read, zeros into a stage nobody reads
+    ob.copy(kt + 1, nxt + kOpB);
+    float fa[2][2][4], fb[2][2][4];  // one chunk pair ahead
+    oa.frags(cur, ra, 0, fa[0]);
+    ob.frags(cur + kOpB, rb, 0, fb[0]);
+    // Keeps the copies up here (the scheduler sank the last one to its wait) and each chunk pair's
+    // reads ahead of the products they run under.
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (c < 3) {
+        oa.frags(cur, ra, c + 1, fa[(c + 1) & 1]);
+        ob.frags(cur + kOpB, rb, c + 1, fb[(c + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma2(fa[c & 1][i][s], fb[c & 1][j][s], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    copies_landed();
+  };
+  oa.copy(0, s0);
+  ob.copy(0, s0 + kOpB);
+  copies_landed();
+  for (int kt = 0; kt < nk; kt += 2) {
+    stage(kt, s0, s1);
+    if (kt + 1 < nk) stage(kt + 1, s1, s0);
+  }
+}
+
 __device__ __forceinline__ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+// Head kinds of the kernels below: dense (any hidden dim), 4-bit, dense on the copied-tile core.
+constexpr int kDense = 0, kQ4 = 1, kCopied = 2;
+template <int KIND>
+constexpr int kStage0 = KIND == kCopied ? 2 * kOpB : 4 * kTileFloats * 4;
+template <int KIND>
+constexpr int kStage1 = KIND == kCopied ? 2 * kOpB : 16;
 
 // ------------------------------------------------------------------------------------------
 // LCE forward: workgroup (128-token tile, vocab split) walks the split's 128-column vocab tiles;
@@ -205,12 +348,15 @@ __device__ __forceinline__ bool aligned16(const void* p) { return ((uintptr_t)p 
 // token, merged with lane ^ 32 and the other vocab-half wave at the end into part_m/part_s
 // [split][N] (log2 domain), which the finalize merges.
 // ------------------------------------------------------------------------------------------
-template <int Q4>
-__global__ __launch_bounds__(256) void lce32_fwd_kernel(const float* __restrict__ H, const float* __restrict__ W,
+template <int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void lce32_fwd_kernel(const float* __restrict__ H, const float* __restrict__ W,
                                                         const uint32_t* __restrict__ Wq, const float* __restrict__ Sc,
                                                         const float* __restrict__ Bi, int N, int D, int V, int nsplit,
                                                         float* __restrict__ part_m, float* __restrict__ part_s) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * kTileFloats];
+  __shared__ __attribute__((aligned(1024))) char s0[kStage0<KIND>];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage1<KIND>];
+  float* lds = reinterpret_cast<float*>(s0);
   const int t0 = blockIdx.x * kT, split = blockIdx.y;
   const int vtiles = (V + kT - 1) / kT;
   const int per = (vtiles + nsplit - 1) / nsplit;
@@ -221,7 +367,9 @@ __global__ __launch_bounds__(256) void lce32_fwd_kernel(const float* __restrict_
   for (int vt = vt0; vt < vt1; ++vt) {
     const int v0 = vt * kT;
     f32x16 acc[2][2];
-    if constexpr (Q4) {
+    if constexpr (KIND == kCopied) {
+      gemm128_copied(RowOp(W + (long)v0 * D, D, V - v0, D), RowOp(H + (long)t0 * D, D, N - t0, D), D, s0, s1, acc);
+    } else if constexpr (KIND == kQ4) {
       Q4RowSrc wa_{Q4Geom{Wq, Sc, Bi, D}, v0, V - v0, D};
       gemm128(wa_, hb, D, lds, acc);
     } else {
@@ -319,21 +467,39 @@ __global__ __launch_bounds__(256) void lce32_finalize_kernel(const float* __rest
 
 // Gradient tile of the backward: C[t][v] = H_t . W_v for rows [row0, row0 + nrows) and the chunk's
 // columns [c0, c0 + ncols); G[t][v - c0] = (exp(C - lse_t) - [v == y_t]) * coef_t in fp32, coef_t =
-// d_nll[t] (0 for ignored rows), 0 past the vocab end.
-template <int Q4>
-__global__ __launch_bounds__(256) void lce32_bwd_g_kernel(const float* __restrict__ H, const float* __restrict__ W,
+// d_nll[t] (0 for ignored rows), 0 past the vocab end (up to a multiple of 4 columns, which the dH
+// product reads).
+template <int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void lce32_bwd_g_kernel(const float* __restrict__ H, const float* __restrict__ W,
                                                           const uint32_t* __restrict__ Wq, const float* __restrict__ Sc,
                                                           const float* __restrict__ Bi, const int64_t* __restrict__ targets,
                                                           const float* __restrict__ lse, const float* __restrict__ dnll,
                                                           int D, int V, long long ignore_index, int row0, int nrows,
                                                           int c0, int ncols, float* __restrict__ G, long ldg) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * kTileFloats];
+  __shared__ __attribute__((aligned(1024))) char s0[kStage0<KIND>];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage1<KIND>];
+  float* lds = reinterpret_cast<float*>(s0);
   const int tt = blockIdx.x * kT, vv = blockIdx.y * kT;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wa = w & 1, wb = w >> 1, h = lane >> 5;
   RowSrc hs{H + (long)(row0 + tt) * D, D, nrows - tt, D, aligned16(H) && D % 4 == 0};
   const int v0 = c0 + vv;
+  // Per row: coefficient, log2-domain lse and the target's column in the chunk (-1: none), fetched ahead
+  // of the product (it has barriers between these writes and the reads below).
+  __shared__ float rcoef[kT], rl2[kT];
+  __shared__ int ry[kT];
+  if (threadIdx.x < kT) {
+    const int t = row0 + tt + threadIdx.x;
+    const bool ok = tt + (int)threadIdx.x < nrows;
+    const long long y = ok ? targets[t] : -1;
+    rcoef[threadIdx.x] = ok && y != ignore_index ? dnll[t] : 0.f;
+    rl2[threadIdx.x] = ok ? lse[t] * kLog2e : 0.f;
+    ry[threadIdx.x] = y >= c0 && y - c0 < ncols ? (int)(y - c0) : -1;
+  }
   f32x16 acc[2][2];
-  if constexpr (Q4) {
+  if constexpr (KIND == kCopied) {
+    gemm128_copied(RowOp(H + (long)(row0 + tt) * D, D, nrows - tt, D), RowOp(W + (long)v0 * D, D, V - v0, D), D, s0, s1, acc);
+  } else if constexpr (KIND == kQ4) {
     Q4RowSrc ws{Q4Geom{Wq, Sc, Bi, D}, v0, V - v0, D};
     gemm128(hs, ws, D, lds, acc);
   } else {
@@ -344,44 +510,39 @@ __global__ __launch_bounds__(256) void lce32_bwd_g_kernel(const float* __restric
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int tl = tt + 64 * wa + 32 * i + rrow(r, h);
+      const int rl = 64 * wa + 32 * i + rrow(r, h), tl = tt + rl;
       if (tl >= nrows) continue;
-      const int t = row0 + tl;
-      const long long y = targets[t];
-      const float coef = (y == ignore_index) ? 0.f : dnll[t];
-      const float l2 = lse[t] * kLog2e;
+      const float coef = rcoef[rl], l2 = rl2[rl];
+      const int y = ry[rl];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int vl = vv + 64 * wb + 32 * j + (lane & 31);
-        if (vl >= ncols) continue;
-        const int v = c0 + vl;
+        if (vl >= ((ncols + 3) & ~3)) continue;
         float g = 0.f;
-        if (v < V) {
+        if (c0 + vl < V) {
           const float p = fast_exp2(__builtin_fmaf(acc[i][j][r], kLog2e, -l2));
-          g = (p - ((long long)v == y ? 1.f : 0.f)) * coef;
+          g = (p - (vl == y ? 1.f : 0.f)) * coef;
         }
         G[(long)tl * ldg + vl] = g;
       }
     }
 }
 
-// C[M][N] (+)= A . B^T, tile (blockIdx.x: 128 rows of C, blockIdx.y: 128 columns); ACC adds to C.
-template <class SA, class SB, bool ACC>
-__device__ __forceinline__ void gemm_store(const SA& sa, const SB& sb, int K, int M, int N, float* __restrict__ C,
-                                           long ldc, float* lds) {
+// Stores (ACC: adds) a product's tile to C[M][N]: blockIdx.x: 128 rows, blockIdx.y: 128 columns. PA, PB: the
+// operands' order of rows within a wave's 64 (the register-staged sources have RowOp's).
+template <bool ACC, class PA = RowOp, class PB = RowOp>
+__device__ __forceinline__ void store_tile(const f32x16 (&acc)[2][2], int M, int N, float* __restrict__ C, long ldc) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wa = w & 1, wb = w >> 1, h = lane >> 5;
-  f32x16 acc[2][2];
-  gemm128(sa, sb, K, lds, acc);
   const int m0 = blockIdx.x * kT, n0 = blockIdx.y * kT;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int m = m0 + 64 * wa + 32 * i + rrow(r, h);
+      const int m = m0 + 64 * wa + PA::pos(i, rrow(r, h));
       if (m >= M) continue;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int n = n0 + 64 * wb + 32 * j + (lane & 31);
+        const int n = n0 + 64 * wb + PB::pos(j, lane & 31);
         if (n >= N) continue;
         float* c = C + (long)m * ldc + n;
         *c = ACC ? *c + acc[i][j][r] : acc[i][j][r];
@@ -395,23 +556,34 @@ __device__ __forceinline__ void gemm_store(const SA& sa, const SB& sb, int K, in
 // one part the tile goes to dH (written by the first chunk, accumulated by the others); with several,
 // each part's tile goes to its own fp32 slice part_out[z] and lce32_dh_reduce_kernel sums them in
 // part order.
-template <int Q4, bool ACC>
-__global__ __launch_bounds__(256) void lce32_dh_kernel(const float* __restrict__ G, long ldg, const float* __restrict__ W,
+template <int KIND, bool ACC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void lce32_dh_kernel(const float* __restrict__ G, long ldg, const float* __restrict__ W,
                                                        const uint32_t* __restrict__ Wq, const float* __restrict__ Sc,
                                                        const float* __restrict__ Bi, int D, int c0, int kcols, int per,
                                                        int nrows, float* __restrict__ dH) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * kTileFloats];
+  __shared__ __attribute__((aligned(1024))) char s0[kStage0<KIND>];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage1<KIND>];
+  float* lds = reinterpret_cast<float*>(s0);
   const int m0 = blockIdx.x * kT, n0 = blockIdx.y * kT;
   const int k0 = blockIdx.z * per;
   const int kn = (kcols - k0 < per) ? kcols - k0 : per;
   float* out = dH + (long)blockIdx.z * nrows * D;
-  RowSrc ga{G + (long)m0 * ldg + k0, ldg, nrows - m0, kn, ldg % 4 == 0};
-  if constexpr (Q4) {
-    Q4ColSrc wb{Q4Geom{Wq, Sc, Bi, D}, (long)c0 + k0, D - n0, kn, n0};
-    gemm_store<RowSrc, Q4ColSrc, ACC>(ga, wb, kn, nrows, D, out, D, lds);
+  f32x16 acc[2][2];
+  if constexpr (KIND == kCopied) {
+    gemm128_copied(RowOp(G + (long)m0 * ldg + k0, ldg, nrows - m0, kn), ColOp(W + (long)(c0 + k0) * D + n0, D, D - n0, kn),
+                   kn, s0, s1, acc);
+    store_tile<ACC, RowOp, ColOp>(acc, nrows, D, out, D);
   } else {
-    ColSrc wb{W + (long)(c0 + k0) * D + n0, D, D - n0, kn, aligned16(W) && D % 4 == 0};
-    gemm_store<RowSrc, ColSrc, ACC>(ga, wb, kn, nrows, D, out, D, lds);
+    RowSrc ga{G + (long)m0 * ldg + k0, ldg, nrows - m0, kn, ldg % 4 == 0};
+    if constexpr (KIND == kQ4) {
+      Q4ColSrc wb{Q4Geom{Wq, Sc, Bi, D}, (long)c0 + k0, D - n0, kn, n0};
+      gemm128(ga, wb, kn, lds, acc);
+    } else {
+      ColSrc wb{W + (long)(c0 + k0) * D + n0, D, D - n0, kn, aligned16(W) && D % 4 == 0};
+      gemm128(ga, wb, kn, lds, acc);
+    }
+    store_tile<ACC>(acc, nrows, D, out, D);
   }
 }
 
@@ -428,13 +600,23 @@ __global__ __launch_bounds__(256) void lce32_dh_reduce_kernel(const float* __res
 
 // dW[v][d] = sum_t G[t][v] H[t][d] for one chunk's vocab rows (all tokens): A = G read k-major
 // (k = t), B = H read k-major.
-__global__ __launch_bounds__(256) void lce32_dw_kernel(const float* __restrict__ G, long ldg, const float* __restrict__ H,
+template <int KIND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void lce32_dw_kernel(const float* __restrict__ G, long ldg, const float* __restrict__ H,
                                                        int N, int D, int vrows, float* __restrict__ dW) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * kTileFloats];
+  __shared__ __attribute__((aligned(1024))) char s0[kStage0<KIND>];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage1<KIND>];
   const int m0 = blockIdx.x * kT, n0 = blockIdx.y * kT;
-  ColSrc ga{G + m0, ldg, vrows - m0, N, ldg % 4 == 0};
-  ColSrc hb{H + n0, D, D - n0, N, aligned16(H) && D % 4 == 0};
-  gemm_store<ColSrc, ColSrc, false>(ga, hb, N, vrows, D, dW, D, lds);
+  f32x16 acc[2][2];
+  if constexpr (KIND == kCopied) {
+    gemm128_copied(ColOp(G + m0, ldg, (int)ldg - m0, N), ColOp(H + n0, D, D - n0, N), N, s0, s1, acc);
+    store_tile<false, ColOp, ColOp>(acc, vrows, D, dW, D);
+  } else {
+    ColSrc ga{G + m0, ldg, vrows - m0, N, ldg % 4 == 0};
+    ColSrc hb{H + n0, D, D - n0, N, aligned16(H) && D % 4 == 0};
+    gemm128(ga, hb, N, reinterpret_cast<float*>(s0), acc);
+    store_tile<false>(acc, vrows, D, dW, D);
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -470,23 +652,6 @@ constexpr int kPos = 32;  // positions per LDS tile
 __device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ void copies_landed() {
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  asm volatile("s_barrier" ::: "memory");
-}
-
-// One global -> LDS copy of a wave: 16 (4) bytes per lane from src + voff (lanes past `bytes` get zeros)
-// to dst + 16 lane (4 lane), dst wave-uniform.
-__device__ __forceinline__ void lds_copy16(const float* src, int bytes, char* dst, uint32_t voff) {
-  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, 0, 0, 0);
-}
-__device__ __forceinline__ void lds_copy4(const float* src, int bytes, char* dst, uint32_t voff) {
-  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, bytes, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, voff, 0, 0, 0);
-}
-
 template <int DH>
 struct ALay {
   static constexpr int kRowB = DH == 64 ? 256 : 512;  // 96: chunks 24-31 of a row stay empty (zeros)
@@ -934,14 +1099,19 @@ int lce32_fwd_nsplit(long N, long V) {
   return ns < 1 ? 1 : (int)ns;
 }
 
+// The copied-tile core takes dense operands whose rows start at multiples of 16 bytes (the entry points
+// check the bases) and whose 128-row tiles stay below the 31-bit offsets of a copy.
+static bool copied_tiles(long d, long ld) { return d % 4 == 0 && ld % 4 == 0 && d < (1L << 21) && ld < (1L << 21); }
+
 hipError_t launch_lce32_fwd(const LceHead32& h, const float* H, const int64_t* targets, int N, int D, int V,
                             long long ignore_index, float* nll, float* lse, float* tgt, float* ws, hipStream_t st) {
   const int ns = lce32_fwd_nsplit(N, V);
   float* pm = ws;
   float* ps = ws + (long)ns * N;
   dim3 grid((N + kT - 1) / kT, ns), block(256);
-  if (h.q4) hipLaunchKernelGGL(lce32_fwd_kernel<1>, grid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, N, D, V, ns, pm, ps);
-  else hipLaunchKernelGGL(lce32_fwd_kernel<0>, grid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, N, D, V, ns, pm, ps);
+  if (h.q4) hipLaunchKernelGGL(lce32_fwd_kernel<kQ4>, grid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, N, D, V, ns, pm, ps);
+  else if (copied_tiles(D, D)) hipLaunchKernelGGL(lce32_fwd_kernel<kCopied>, grid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, N, D, V, ns, pm, ps);
+  else hipLaunchKernelGGL(lce32_fwd_kernel<kDense>, grid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, N, D, V, ns, pm, ps);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   dim3 fgrid((N + 3) / 4);
@@ -970,12 +1140,14 @@ hipError_t launch_lce32_bwd(const LceHead32& h, const float* H, const int64_t* t
                             const float* dnll, int N, int D, int V, long long ignore_index, int chunk, float* dH,
                             float* dW, float* Gbuf, hipStream_t st) {
   const long ldg = (long)chunk + 4;
+  const bool copied = copied_tiles(D, ldg);
   dim3 block(256);
   for (int c0 = 0; c0 < V; c0 += chunk) {
     const int kc = (V - c0 < chunk) ? V - c0 : chunk;
     dim3 ggrid((N + kT - 1) / kT, (kc + kT - 1) / kT);
-    if (h.q4) hipLaunchKernelGGL(lce32_bwd_g_kernel<1>, ggrid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, targets, lse, dnll, D, V, ignore_index, 0, N, c0, kc, Gbuf, ldg);
-    else hipLaunchKernelGGL(lce32_bwd_g_kernel<0>, ggrid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, targets, lse, dnll, D, V, ignore_index, 0, N, c0, kc, Gbuf, ldg);
+    if (h.q4) hipLaunchKernelGGL(lce32_bwd_g_kernel<kQ4>, ggrid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, targets, lse, dnll, D, V, ignore_index, 0, N, c0, kc, Gbuf, ldg);
+    else if (copied) hipLaunchKernelGGL(lce32_bwd_g_kernel<kCopied>, ggrid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, targets, lse, dnll, D, V, ignore_index, 0, N, c0, kc, Gbuf, ldg);
+    else hipLaunchKernelGGL(lce32_bwd_g_kernel<kDense>, ggrid, block, 0, st, H, h.w, h.wq, h.sc, h.bi, targets, lse, dnll, D, V, ignore_index, 0, N, c0, kc, Gbuf, ldg);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const bool acc = c0 > 0;
@@ -984,16 +1156,20 @@ hipError_t launch_lce32_bwd(const LceHead32& h, const float* H, const int64_t* t
     dim3 hgrid((N + kT - 1) / kT, (D + kT - 1) / kT, np);
     if (np == 1) {
       if (h.q4) {
-        if (acc) hipLaunchKernelGGL((lce32_dh_kernel<1, true>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
-        else hipLaunchKernelGGL((lce32_dh_kernel<1, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+        if (acc) hipLaunchKernelGGL((lce32_dh_kernel<kQ4, true>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+        else hipLaunchKernelGGL((lce32_dh_kernel<kQ4, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+      } else if (copied) {
+        if (acc) hipLaunchKernelGGL((lce32_dh_kernel<kCopied, true>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+        else hipLaunchKernelGGL((lce32_dh_kernel<kCopied, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
       } else {
-        if (acc) hipLaunchKernelGGL((lce32_dh_kernel<0, true>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
-        else hipLaunchKernelGGL((lce32_dh_kernel<0, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+        if (acc) hipLaunchKernelGGL((lce32_dh_kernel<kDense, true>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
+        else hipLaunchKernelGGL((lce32_dh_kernel<kDense, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, dH);
       }
     } else {
       float* parts = Gbuf + (long)N * ldg;   // after the gradient tile: [np][N][D]
-      if (h.q4) hipLaunchKernelGGL((lce32_dh_kernel<1, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, parts);
-      else hipLaunchKernelGGL((lce32_dh_kernel<0, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, parts);
+      if (h.q4) hipLaunchKernelGGL((lce32_dh_kernel<kQ4, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, parts);
+      else if (copied) hipLaunchKernelGGL((lce32_dh_kernel<kCopied, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, parts);
+      else hipLaunchKernelGGL((lce32_dh_kernel<kDense, false>), hgrid, block, 0, st, Gbuf, ldg, h.w, h.wq, h.sc, h.bi, D, c0, kc, per, N, parts);
       e = hipGetLastError();
       if (e != hipSuccess) return e;
       const long count = (long)N * D;
@@ -1005,7 +1181,8 @@ hipError_t launch_lce32_bwd(const LceHead32& h, const float* H, const int64_t* t
     if (e != hipSuccess) return e;
     if (dW) {
       dim3 wgrid((kc + kT - 1) / kT, (D + kT - 1) / kT);
-      hipLaunchKernelGGL(lce32_dw_kernel, wgrid, block, 0, st, Gbuf, ldg, H, N, D, kc, dW + (long)c0 * D);
+      if (copied) hipLaunchKernelGGL(lce32_dw_kernel<kCopied>, wgrid, block, 0, st, Gbuf, ldg, H, N, D, kc, dW + (long)c0 * D);
+      else hipLaunchKernelGGL(lce32_dw_kernel<kDense>, wgrid, block, 0, st, Gbuf, ldg, H, N, D, kc, dW + (long)c0 * D);
       e = hipGetLastError();
       if (e != hipSuccess) return e;
     }

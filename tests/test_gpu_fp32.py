@@ -350,6 +350,16 @@ def _attn_check_rel(got, q, k, v, do, scale, *, causal=True, sid=None, tag=""):
     assert all(x < 1e-5 for x in e.values()), e
 
 
+# Edges of the copied-tile core: hidden dims around its 32-deep stages (and 30, which it leaves to the
+# register-staged one), token counts and vocabularies around its 128-row tiles, vocabularies that end inside a
+# 4-column chunk of the gradient tile, and a hidden dim past one 128-column tile.
+@pytest.mark.parametrize(("kind", "n", "d", "v"), [
+    ("trainable", 1, 4, 5), ("trainable", 127, 28, 129), ("trainable", 129, 36, 1023), ("dense", 128, 60, 127),
+    ("trainable", 31, 132, 641), ("dense", 257, 64, 2050), ("trainable", 64, 30, 131), ("dense", 33, 260, 1)])
+def test_lce_fp32_tile_edges(kind, n, d, v):
+    test_lce_fp32_random(kind, n, d, v)
+
+
 @pytest.mark.parametrize(("b", "hq", "hkv", "s", "d", "causal"), RAND_ATT)
 def test_attention_fp32_random(b, hq, hkv, s, d, causal):
     print(f"[attention fp32 random b={b} hq={hq} hkv={hkv} s={s} d={d} causal={causal}]", flush=True)
