@@ -89,6 +89,16 @@ def test_causal_parity_edge_lengths(shape):
             assert rel_l2(got, want) <= 1e-2
 
 
+# Workgroups of the dK/dV pass with 0 to 6 tiles: up to 40 (head, 64-query tile) items over 8 splits. Its loop
+# runs three tiles at a time and finishes the last one by itself.
+@pytest.mark.parametrize("s", [64, 130, 257, 385, 449, 600])
+@pytest.mark.parametrize("causal", [True, False])
+def test_dkv_tile_counts(s, causal):
+    q, k, v, do = attn_inputs(1, 4, 1, s, 64, seed=s)
+    scale = 0.125
+    _check(_run_kernel(q, k, v, do, scale, causal=causal), q, k, v, do, scale, causal=causal)
+
+
 @pytest.mark.parametrize("shape", [(1, 8, 2, 1100, 128), (1, 4, 1, 130, 96), (1, 4, 2, 257, 64)])
 def test_causal_parity_rising_maxima(shape):
     """Scores with a large spread whose row maxima keep rising along the keys, so the online
