@@ -377,6 +377,23 @@ int mtp_lce_bwd(const void* hidden, const void* w, const void* w_t, const uint32
   return ok();
 }
 
+int mtp_lce_mean(const float* nll, const int64_t* targets, int64_t n, int64_t ignore_index, float* mean, float* count,
+                 void* stream) {
+  if (n < 1 || n > kMaxDim) return fail(MTP_ERR_INPUT, "n must be in [1, 2^31) (got n=%lld)", (long long)n);
+  if (!nll || !targets || !mean || !count) return fail(MTP_ERR_INPUT, "nll, targets, mean and count must be non-null");
+  hipError_t e = mtp::launch_lce_mean(nll, targets, (long)n, (long long)ignore_index, mean, count, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(MTP_ERR_RUNTIME, "lce mean launch failed: %s", hipGetErrorString(e));
+  return ok();
+}
+
+int mtp_lce_mean_bwd(const float* d_mean, const float* count, int64_t n, float* d_nll, void* stream) {
+  if (n < 1 || n > kMaxDim) return fail(MTP_ERR_INPUT, "n must be in [1, 2^31) (got n=%lld)", (long long)n);
+  if (!d_mean || !count || !d_nll) return fail(MTP_ERR_INPUT, "d_mean, count and d_nll must be non-null");
+  hipError_t e = mtp::launch_lce_mean_bwd(d_mean, count, (long)n, d_nll, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(MTP_ERR_RUNTIME, "lce mean backward launch failed: %s", hipGetErrorString(e));
+  return ok();
+}
+
 int mtp_attn_fwd(const void* q, const void* k, const void* v, int64_t b, int64_t hq, int64_t hkv, int64_t s,
                  int64_t dh, float scale, int32_t causal, const int32_t* seg_id, const int32_t* seg_start, void* o,
                  float* lse, void* stream) {

@@ -1803,9 +1803,7 @@ constexpr long kFwdWaves = 1;
 // forward's partials [2][splits][N] fp32 never exceed 4 MiB for N <= 524288. (A count that only just
 // overflows one round, e.g. 48 row tiles x 6 splits = 288 workgroups, would run two rounds of one
 // split's tiles each.)
-static int lce_nsplit(long N, long V, int per_cu) {
-  const long rtiles = (N + kTile - 1) / kTile;
-  const long vtiles = (V + kTile - 1) / kTile;
+static int lce_nsplit_plan(long rtiles, long vtiles, int per_cu) {
   const long slots = (long)per_cu * kNumCU;
   long top = vtiles < 1024 ? vtiles : 1024;
   if (top > 2048 / rtiles) top = 2048 / rtiles > 1 ? 2048 / rtiles : 1;
@@ -1821,6 +1819,20 @@ static int lce_nsplit(long N, long V, int per_cu) {
   for (long ns = 1; ns <= top; ++ns)
     if (cost(ns) * 100 <= least * 105) return (int)ns;
   return 1;
+}
+// The plan of a thread's latest shapes: each entry point asks for its shape's several times, and the
+// search over up to 1024 counts is 20 us of host time each.
+static int lce_nsplit(long N, long V, int per_cu) {
+  struct Plan {
+    long rtiles, vtiles;
+    int per_cu, ns;
+  };
+  thread_local Plan plans[16] = {};
+  const long rtiles = (N + kTile - 1) / kTile, vtiles = (V + kTile - 1) / kTile;
+  Plan& p = plans[(rtiles * 7 + vtiles) & 15];
+  if (p.ns == 0 || p.rtiles != rtiles || p.vtiles != vtiles || p.per_cu != per_cu)
+    p = Plan{rtiles, vtiles, per_cu, lce_nsplit_plan(rtiles, vtiles, per_cu)};
+  return p.ns;
 }
 
 // Parts of the dH product's vocab contraction (1 = none) for `rows` rows, D columns and `ktiles`
@@ -1947,6 +1959,60 @@ hipError_t launch_lce_fwd(const LceHead& h, const bf16_t* H, const int64_t* targ
     hipLaunchKernelGGL(lce_fwd_finalize_kernel<0>, fgrid, fblock, 0, stream, H, h.w, h.wq, h.sc, h.bi, targets, N,
                        D, V, ns, pm, ps, ignore_index, nll, lse, tgt);
   }
+  return hipGetLastError();
+}
+
+// Mean loss of the tokens that are not ignored: mean = sum(nll) / max(count, 1), summed in 64 bits (an
+// ignored token's nll is 0), and the count. One workgroup: 8192 tokens are 96 KiB, about 4 us; as
+// torch operators (compare, two sums, clamp, convert, divide) it is six launches.
+__global__ __launch_bounds__(1024) void lce_mean_kernel(const float* __restrict__ nll,
+                                                        const int64_t* __restrict__ targets, long n,
+                                                        long long ignore_index, float* __restrict__ mean,
+                                                        float* __restrict__ count) {
+  __shared__ double sums[16];
+  __shared__ int counts[16];
+  double s = 0.0;
+  int c = 0;
+  for (long i = threadIdx.x; i < n; i += 1024) {
+    s += (double)nll[i];
+    c += targets[i] != ignore_index;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    s += __shfl_xor(s, o, 64);
+    c += __shfl_xor(c, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sums[threadIdx.x >> 6] = s;
+    counts[threadIdx.x >> 6] = c;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) {
+      s += sums[w];
+      c += counts[w];
+    }
+    if (c < 1) c = 1;
+    *mean = (float)(s / (double)c);
+    *count = (float)c;
+  }
+}
+
+// d_nll[i] = d_mean / count for every token (the loss backward leaves ignored ones out).
+__global__ __launch_bounds__(256) void lce_mean_bwd_kernel(const float* __restrict__ d_mean,
+                                                           const float* __restrict__ count, long n,
+                                                           float* __restrict__ d_nll) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) d_nll[i] = *d_mean / *count;
+}
+
+hipError_t launch_lce_mean(const float* nll, const int64_t* targets, long n, long long ignore_index, float* mean,
+                           float* count, hipStream_t stream) {
+  hipLaunchKernelGGL(lce_mean_kernel, dim3(1), dim3(1024), 0, stream, nll, targets, n, ignore_index, mean, count);
+  return hipGetLastError();
+}
+hipError_t launch_lce_mean_bwd(const float* d_mean, const float* count, long n, float* d_nll, hipStream_t stream) {
+  hipLaunchKernelGGL(lce_mean_bwd_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, d_mean, count, n, d_nll);
   return hipGetLastError();
 }
 

@@ -61,6 +61,10 @@ hipError_t launch_lce_bwd(const LceHead& h, const bf16_t* H, const int64_t* targ
                           bf16_t* dH, bf16_t* dW, bf16_t* Gbuf, float* acc32, float* parts, bf16_t* stage,
                           hipStream_t stream);
 
+hipError_t launch_lce_mean(const float* nll, const int64_t* targets, long n, long long ignore_index, float* mean,
+                           float* count, hipStream_t stream);
+hipError_t launch_lce_mean_bwd(const float* d_mean, const float* count, long n, float* d_nll, hipStream_t stream);
+
 struct AttnShape {
   int b, hq, hkv, s, dh;
   float scale;

@@ -73,6 +73,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "mtp_lce_bwd": (ctypes.c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                    _i64, _i64, _i64, _i32, _i64, _c_void_p, _c_void_p, _c_void_p,
                                    _c_void_p, _i64, _i64, _c_void_p, _size, _c_void_p]),
+    "mtp_lce_mean": (ctypes.c_int, [_c_void_p, _c_void_p, _i64, _i64, _c_void_p, _c_void_p, _c_void_p]),
+    "mtp_lce_mean_bwd": (ctypes.c_int, [_c_void_p, _c_void_p, _i64, _c_void_p, _c_void_p]),
     "mtp_attn_fwd": (ctypes.c_int, [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _i64, _i64,
                                     _f32, _i32, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
     "mtp_attn_bwd_workspace_bytes": (_size, [_i64, _i64, _i64, _i64, _i64]),
@@ -157,7 +159,8 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # current_stream(t.device).cuda_stream without the Stream object it builds on every call
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def on_device(t: torch.Tensor):

@@ -215,6 +215,9 @@ class _KernelAttention(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, o, lse, seg_id, seg_start)
         ctx.scale, ctx.causal = scale, causal
         ctx.mark_non_differentiable(lse)
+        # No zeros in the place of L's gradient, which has none: autograd would fill a tensor for it in
+        # every backward.
+        ctx.set_materialize_grads(False)
         return o, lse
 
     @staticmethod
@@ -222,7 +225,8 @@ class _KernelAttention(torch.autograd.Function):
         VJP_CALLS["flash_attention"] = VJP_CALLS.get("flash_attention", 0) + 1
         VJP_CALLS["flash_attention_kernel_bwd"] = VJP_CALLS.get("flash_attention_kernel_bwd", 0) + 1
         q, k, v, o, lse, seg_id, seg_start = ctx.saved_tensors
-        dq, dk, dv = kernel_backward(q, k, v, o, lse, d_o.contiguous(), scale=ctx.scale, seg_id=seg_id,
+        d_o = torch.zeros_like(o) if d_o is None else d_o.contiguous()
+        dq, dk, dv = kernel_backward(q, k, v, o, lse, d_o, scale=ctx.scale, seg_id=seg_id,
                                      seg_start=seg_start, causal=ctx.causal)
         return dq, dk, dv, None, None, None, None
 

@@ -127,18 +127,28 @@ def resolve_impl(*, head: HeadRef, dtype: torch.dtype, n: int, impl: str = "auto
     (the MI355X analogue of the reference's mlx version gate)."""
     if n <= 0:
         raise LossInputError(f"n must be positive (hidden's row count); got n={n}")
-    if impl == "chunked":
-        return Resolution(impl="chunked", row_tiles=None, provisional=False, reason="explicit impl='chunked' opt-in")
-    if impl == "naive":
-        return Resolution(impl="naive", row_tiles=None, provisional=False, reason="explicit impl='naive' opt-in")
-    if impl not in ("auto", "kernel"):
-        raise LossInputError(f"unknown impl {impl!r}; expected one of 'auto', 'kernel', 'chunked', 'naive'")
-    _require_kernel_supported(head=head, dtype=dtype)
-    _compat.check_device_verified(allow_unverified=allow_unverified_mlx, error=UnsupportedHeadError)
+    resolved = _resolve(head=head, dtype=dtype, impl=impl, allow_unverified_mlx=allow_unverified_mlx)
+    if resolved != "kernel":
+        return Resolution(impl=resolved, row_tiles=None, provisional=False, reason=f"explicit impl='{resolved}' opt-in")
     plan = _plan.lce_plan(n=n, v=_head_v(head))
     reason = (f"kernel: {_KERNEL_ROW_TILE}-row x 256-vocab MFMA tiles, {plan.fwd_splits} vocab splits "
               f"for n={n}")
     return Resolution(impl="kernel", row_tiles=_KERNEL_ROW_TILE, provisional=False, reason=reason)
+
+
+def _resolve(*, head: HeadRef, dtype: torch.dtype, impl: str,
+             allow_unverified_mlx: bool) -> Literal["kernel", "chunked", "naive"]:
+    """resolve_impl's choice and refusals, without the launch plan that its reason quotes (the loss asks
+    on every call)."""
+    if impl == "chunked":
+        return "chunked"
+    if impl == "naive":
+        return "naive"
+    if impl not in ("auto", "kernel"):
+        raise LossInputError(f"unknown impl {impl!r}; expected one of 'auto', 'kernel', 'chunked', 'naive'")
+    _require_kernel_supported(head=head, dtype=dtype)
+    _compat.check_device_verified(allow_unverified=allow_unverified_mlx, error=UnsupportedHeadError)
+    return "kernel"
 
 
 def _head_v(head: HeadRef) -> int:
@@ -316,12 +326,15 @@ def _forward_stage_bytes(lib, n: int, d: int, v: int, head_kind: int, f32: bool)
 
 
 class _KernelLCE(torch.autograd.Function):
-    """Forward: mtp_lce_fwd -> (nll, lse, tgt). Backward: mtp_lce_bwd from the saved lse only; it also
-    returns dL/dW when the dense head is an input that requires grad (trainable head). fp32 hidden
-    states run the fp32 entry points (mtp_lce_fwd_f32 / mtp_lce_bwd_f32)."""
+    """Forward: mtp_lce_fwd -> (nll, lse, tgt), or with `mean` (mean, lse, tgt), nll's mean over the tokens
+    that are not ignored (mtp_lce_mean: one launch, and one in the backward, where torch operators take
+    six and five). Backward: mtp_lce_bwd from the saved lse only; it also returns dL/dW when the dense
+    head is an input that requires grad (trainable head). fp32 hidden states run the fp32 entry points
+    (mtp_lce_fwd_f32 / mtp_lce_bwd_f32)."""
 
     @staticmethod
-    def forward(ctx, hidden2, targets2, w, w_q, scales, biases, head_kind, ignore_index, bwd_chunk, owner=None):
+    def forward(ctx, hidden2, targets2, w, w_q, scales, biases, head_kind, ignore_index, bwd_chunk, owner=None,
+                mean=False):
         lib = _native.load()
         n, d = hidden2.shape
         v = w.shape[0] if head_kind == _native.HEAD_DENSE else w_q.shape[0]
@@ -345,21 +358,33 @@ class _KernelLCE(torch.autograd.Function):
                      targets2.data_ptr(), n, d, v, fwd_kind, ignore_index, nll.data_ptr(), lse.data_ptr(),
                      tgt.data_ptr(), ws.data_ptr(), ws_bytes, _native.stream_of(hidden2))
         _native.check(rc, domain="loss")
-        ctx.save_for_backward(hidden2, targets2, lse)
+        count = None
+        if mean:
+            nll, count = _mean_nll(lib, nll, targets2, ignore_index)
+        ctx.save_for_backward(hidden2, targets2, lse, count)
         ctx.head = (w, w_q, scales, biases, head_kind, v)
         ctx.ignore_index = ignore_index
         ctx.bwd_chunk = bwd_chunk
         ctx.owner = owner
         ctx.mark_non_differentiable(lse, tgt)
+        ctx.set_materialize_grads(False)   # no zeros filled in the place of lse's and tgt's gradients
         return nll, lse, tgt
 
     @staticmethod
     def backward(ctx, d_nll, _d_lse, _d_tgt):
         VJP_CALLS["kernel"] = VJP_CALLS.get("kernel", 0) + 1
         lib = _native.load()
-        hidden2, targets2, lse = ctx.saved_tensors
+        hidden2, targets2, lse, count = ctx.saved_tensors
         w, w_q, scales, biases, head_kind, v = ctx.head
         n, d = hidden2.shape
+        if d_nll is None:
+            d_nll = torch.zeros_like(lse)
+        elif count is not None:   # the gradient of the mean
+            d_mean, d_nll = d_nll.to(torch.float32), torch.empty_like(lse)
+            with _native.on_device(hidden2):
+                rc = lib.mtp_lce_mean_bwd(d_mean.data_ptr(), count.data_ptr(), n, d_nll.data_ptr(),
+                                          _native.stream_of(hidden2))
+            _native.check(rc, domain="loss")
         d_w = torch.empty_like(w) if (w is not None and ctx.needs_input_grad[2]) else None
         if hidden2.dtype == torch.float32:
             return _f32_backward(lib, ctx, hidden2, targets2, lse, d_nll, d_w)
@@ -393,7 +418,18 @@ class _KernelLCE(torch.autograd.Function):
                                  ctx.ignore_index, lse.data_ptr(), ct.data_ptr(), d_hidden.data_ptr(),
                                  _native.ptr(d_w), chunk, rows, ws.data_ptr(), ws_bytes, _native.stream_of(hidden2))
         _native.check(rc, domain="loss")
-        return d_hidden, None, d_w, None, None, None, None, None, None, None
+        return d_hidden, None, d_w, None, None, None, None, None, None, None, None
+
+
+def _mean_nll(lib, nll, targets2, ignore_index):
+    """(mean, count) of the per-token loss over the tokens that are not ignored, in one launch."""
+    mean = torch.empty((), dtype=torch.float32, device=nll.device)
+    count = torch.empty((), dtype=torch.float32, device=nll.device)
+    with _native.on_device(nll):
+        rc = lib.mtp_lce_mean(nll.data_ptr(), targets2.data_ptr(), nll.shape[0], ignore_index, mean.data_ptr(),
+                              count.data_ptr(), _native.stream_of(nll))
+    _native.check(rc, domain="loss")
+    return mean, count
 
 
 def _f32_backward(lib, ctx, hidden2, targets2, lse, d_nll, d_w):
@@ -416,7 +452,7 @@ def _f32_backward(lib, ctx, hidden2, targets2, lse, d_nll, d_w):
                                  lse.data_ptr(), ct.data_ptr(), d_hidden.data_ptr(), _native.ptr(d_w), chunk,
                                  ws.data_ptr(), ws_bytes, _native.stream_of(hidden2))
     _native.check(rc, domain="loss")
-    return d_hidden, None, d_w, None, None, None, None, None, None, None
+    return d_hidden, None, d_w, None, None, None, None, None, None, None, None
 
 
 def _require_same_device(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor) -> None:
@@ -435,8 +471,9 @@ def _require_same_device(hidden2: torch.Tensor, head: HeadRef, targets2: torch.T
 
 
 def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *, ignore_index: int = -100,
-                         bwd_chunk: int | None = None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(nll, lse, tgt) from the kernel impl, differentiable in hidden2 through `nll` (test/bench seam)."""
+                         bwd_chunk: int | None = None, mean: bool = False) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(nll, lse, tgt) from the kernel impl, differentiable in hidden2 through `nll` (test/bench seam). `mean`:
+    the mean of nll over the tokens that are not ignored in its place."""
     _require_same_device(hidden2, head, targets2)
     h = hidden2.contiguous()
     t = targets2.to(torch.int64).contiguous()
@@ -445,11 +482,11 @@ def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.T
         if not w.is_contiguous():
             raise UnsupportedHeadError("kernel impl needs a contiguous (V, D) head weight")
         return _KernelLCE.apply(h, t, w, None, None, None, _native.HEAD_DENSE, int(ignore_index), int(bwd_chunk or 0),
-                                head.weight)
+                                head.weight, mean)
     sb = torch.float32 if h.dtype == torch.float32 else torch.bfloat16   # the fp32 kernels read fp32 scales
     args = (None, head.w_q.contiguous(), head.scales.to(sb).contiguous(), head.biases.to(sb).contiguous(),
             _native.HEAD_Q4)
-    return _KernelLCE.apply(h, t, *args, int(ignore_index), int(bwd_chunk or 0), head.w_q)
+    return _KernelLCE.apply(h, t, *args, int(ignore_index), int(bwd_chunk or 0), head.w_q, mean)
 
 
 def linear_cross_entropy(
@@ -475,12 +512,14 @@ def linear_cross_entropy(
     leading = tuple(hidden.shape[:-1])
     hidden2 = hidden.reshape(-1, hidden.shape[-1])
     targets2 = targets.reshape(-1)
-    n = hidden2.shape[0]
-    res = resolve_impl(head=head, dtype=hidden2.dtype, n=n, impl=impl, allow_unverified_mlx=allow_unverified_mlx)
-    if res.impl == "naive":
+    resolved = _resolve(head=head, dtype=hidden2.dtype, impl=impl, allow_unverified_mlx=allow_unverified_mlx)
+    if resolved == "naive":
         nll = _naive_nll(hidden2, head, targets2, ignore_index)
-    elif res.impl == "chunked":
+    elif resolved == "chunked":
         nll = _chunked_nll(hidden2, head, targets2, ignore_index, _DEFAULT_CHUNK if chunk_size is None else chunk_size)
     else:
-        nll, _, _ = kernel_forward_parts(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size)
+        nll, _, _ = kernel_forward_parts(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size,
+                                         mean=reduction == "mean")
+        if reduction == "mean":
+            return nll
     return _reduce(nll, reduction=reduction, leading=leading, targets2=targets2, ignore_index=ignore_index)

@@ -197,6 +197,57 @@ def test_trainable_head_dw_ragged_tokens(n, d, v, chunk):
     test_trainable_head_dw_parity(n, d, v, chunk)
 
 
+# One token, around the mean kernel's 1024 threads, several tokens a thread; every token, some and none ignored.
+@pytest.mark.parametrize("n", [1, 1023, 1025, 5000])
+@pytest.mark.parametrize("ignored", [0.0, 0.3, 1.0])
+def test_mean_loss_and_its_gradient(n, ignored):
+    """reduction="mean" against the per-token losses' mean in 64 bits and the gradient of reduction="none"
+    with that mean's cotangent."""
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+
+    h, w, t = lce_inputs(n, 64, 300, seed=n)
+    t = t.clone()
+    t[torch.arange(n) < round(n * ignored)] = IGN
+    if ignored == 0.0:
+        t[t == IGN] = 0
+    head = DenseHead(weight=w.cuda(), trainable=False)
+    hd, td = h.cuda().requires_grad_(True), t.cuda()
+    loss = linear_cross_entropy(hd, head, td)
+    nll = linear_cross_entropy(hd, head, td, reduction="none")
+    count = max(int((t != IGN).sum()), 1)
+    want = float(nll.detach().double().sum() / count)
+    assert loss.shape == () and loss.dtype == torch.float32
+    assert abs(float(loss.detach()) - want) <= 2 ** -23 * abs(want)   # one rounding of the 64-bit mean
+    (dh,) = torch.autograd.grad(loss, hd, torch.tensor(2.0, device="cuda"))
+    (ref,) = torch.autograd.grad(nll, hd, torch.full((n,), 2.0, device="cuda") / count)
+    assert torch.equal(dh, ref)
+
+
+def test_undefined_gradient_is_zero():
+    """A user's autograd node that returns no gradient for the losses or for O: the gradients are zeros."""
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+    from mlx_train_perf.attention import flash_attention
+
+    class Drop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+
+    h, w, t = lce_inputs(40, 64, 300, seed=1)
+    hd = h.cuda().requires_grad_(True)
+    for reduction in ("none", "mean"):
+        loss = linear_cross_entropy(hd, DenseHead(weight=w.cuda(), trainable=False), t.cuda(), reduction=reduction)
+        (dh,) = torch.autograd.grad(Drop.apply(loss).sum(), hd)
+        assert dh.shape == hd.shape and not dh.any()
+    q, k, v = (torch.randn(1, 2, 40, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
+    for g in torch.autograd.grad(Drop.apply(flash_attention(q, k, v, scale=0.125)).sum(), (q, k, v)):
+        assert not g.any()
+
+
 @pytest.mark.parametrize(("v", "d"), [(1027, 192), (300, 64), (5000, 512)])
 def test_head_transpose_exact(v, d):
     """mtp_lce_head_transpose: w_t[:, :v] == w.T bitwise, zero padding up to the row pitch."""
