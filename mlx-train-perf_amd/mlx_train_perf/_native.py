@@ -130,6 +130,43 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+_nodes = None
+
+
+def nodes():
+    """Load (once) and return the extension module with the autograd nodes (csrc/torch_nodes.cpp), bound to
+    the loaded library's entry points; raise if it is absent."""
+    global _nodes
+    if _nodes is not None:
+        return _nodes
+    lib = load()
+    with _lock:
+        if _nodes is None:
+            try:
+                from mlx_train_perf import _mtp_torch
+            except ImportError as e:
+                raise MissingDependencyError(
+                    f"the autograd nodes {Path(__file__).with_name('_mtp_torch.so')} cannot be loaded ({e}); run "
+                    "`python -c \"import __graft_entry__ as g; g.build()\"` from the repository root.") from e
+            from mlx_train_perf.attention import api
+            from mlx_train_perf.core import loss
+            from mlx_train_perf.plan import launch
+
+            _mtp_torch.bind({name: ctypes.cast(getattr(lib, name), _c_void_p).value for name in SIGNATURES}, check)
+            _mtp_torch.bind_attention(api.VJP_CALLS)
+            _mtp_torch.bind_loss(loss.VJP_CALLS, loss._transposed_head, launch.lce_bwd_budget_bytes)
+            _nodes = _mtp_torch
+    return _nodes
+
+
+def plain(*tensors: torch.Tensor) -> bool:
+    """Ordinary tensors outside function transforms, tracing and dispatch modes: the calls that the C++
+    nodes take. The others keep the Python Functions, which refuse or serve them as they always did."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and not torch._C._are_functorch_transforms_active() and torch._C._get_tracing_state() is None
+            and not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0)
+
+
 def gpu_available() -> bool:
     return torch.cuda.is_available()
 

@@ -209,6 +209,8 @@ def kernel_backward(q, k, v, o, lse, d_o, *, scale: float, seg_id=None, seg_star
 
 
 class _KernelAttention(torch.autograd.Function):
+    """The general path; flash_attention runs the C++ node of the same calls on plain tensors."""
+
     @staticmethod
     def forward(ctx, q, k, v, seg_id, seg_start, scale, causal):
         o, lse = kernel_forward(q, k, v, scale=scale, seg_id=seg_id, seg_start=seg_start, causal=causal)
@@ -246,6 +248,9 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale:
                                       validate_segments=validate_segments)
     seg_id, seg_start = (None, None) if segments is None else _seg_args(q, segments.seg_id, segments.seg_start)
     if resolved == "kernel":
+        if _native.plain(q, k, v):
+            return _native.nodes().attention(q.contiguous(), k.contiguous(), v.contiguous(), seg_id, seg_start,
+                                             float(scale), bool(causal))
         o, _ = _KernelAttention.apply(q.contiguous(), k.contiguous(), v.contiguous(), seg_id, seg_start, float(scale),
                                       bool(causal))
         return o

@@ -326,7 +326,8 @@ def _forward_stage_bytes(lib, n: int, d: int, v: int, head_kind: int, f32: bool)
 
 
 class _KernelLCE(torch.autograd.Function):
-    """Forward: mtp_lce_fwd -> (nll, lse, tgt), or with `mean` (mean, lse, tgt), nll's mean over the tokens
+    """The general path; the loss runs the C++ node of the same calls on plain tensors (_kernel_loss).
+    Forward: mtp_lce_fwd -> (nll, lse, tgt), or with `mean` (mean, lse, tgt), nll's mean over the tokens
     that are not ignored (mtp_lce_mean: one launch, and one in the backward, where torch operators take
     six and five). Backward: mtp_lce_bwd from the saved lse only; it also returns dL/dW when the dense
     head is an input that requires grad (trainable head). fp32 hidden states run the fp32 entry points
@@ -470,10 +471,8 @@ def _require_same_device(hidden2: torch.Tensor, head: HeadRef, targets2: torch.T
                                  "needs every input on the same GPU")
 
 
-def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *, ignore_index: int = -100,
-                         bwd_chunk: int | None = None, mean: bool = False) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(nll, lse, tgt) from the kernel impl, differentiable in hidden2 through `nll` (test/bench seam). `mean`:
-    the mean of nll over the tokens that are not ignored in its place."""
+def _kernel_args(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor) -> tuple:
+    """(hidden2, targets2, w, w_q, scales, biases, head_kind, owner) as the kernels read them."""
     _require_same_device(hidden2, head, targets2)
     h = hidden2.contiguous()
     t = targets2.to(torch.int64).contiguous()
@@ -481,12 +480,30 @@ def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.T
         w = head.weight if head.trainable else head.weight.detach()
         if not w.is_contiguous():
             raise UnsupportedHeadError("kernel impl needs a contiguous (V, D) head weight")
-        return _KernelLCE.apply(h, t, w, None, None, None, _native.HEAD_DENSE, int(ignore_index), int(bwd_chunk or 0),
-                                head.weight, mean)
+        return h, t, w, None, None, None, _native.HEAD_DENSE, head.weight
     sb = torch.float32 if h.dtype == torch.float32 else torch.bfloat16   # the fp32 kernels read fp32 scales
-    args = (None, head.w_q.contiguous(), head.scales.to(sb).contiguous(), head.biases.to(sb).contiguous(),
-            _native.HEAD_Q4)
-    return _KernelLCE.apply(h, t, *args, int(ignore_index), int(bwd_chunk or 0), head.w_q, mean)
+    return (h, t, None, head.w_q.contiguous(), head.scales.to(sb).contiguous(), head.biases.to(sb).contiguous(),
+            _native.HEAD_Q4, head.w_q)
+
+
+def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *, ignore_index: int = -100,
+                         bwd_chunk: int | None = None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(nll, lse, tgt) from the kernel impl, differentiable in hidden2 through `nll` (test/bench seam)."""
+    *args, owner = _kernel_args(hidden2, head, targets2)
+    return _KernelLCE.apply(*args, int(ignore_index), int(bwd_chunk or 0), owner)
+
+
+def _kernel_loss(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *, ignore_index: int,
+                 bwd_chunk: int | None, mean: bool) -> torch.Tensor:
+    """nll, or its mean over the tokens that are not ignored: the C++ node of _KernelLCE on plain tensors."""
+    *args, owner = _kernel_args(hidden2, head, targets2)
+    args += [int(ignore_index), int(bwd_chunk or 0), owner, mean]
+    h, _, w, w_q, _, _, kind = args[:7]
+    if not _native.plain(*(x for x in args if isinstance(x, torch.Tensor))):
+        return _KernelLCE.apply(*args)[0]
+    v, d = (w if kind == _native.HEAD_DENSE else w_q).shape[0], h.shape[1]
+    ws_bytes = _forward_stage_bytes(_native.load(), h.shape[0], d, v, kind, h.dtype == torch.float32)
+    return _native.nodes().loss(*args, _native.HEAD_Q4_STAGED if ws_bytes else kind, ws_bytes)
 
 
 def linear_cross_entropy(
@@ -518,8 +535,8 @@ def linear_cross_entropy(
     elif resolved == "chunked":
         nll = _chunked_nll(hidden2, head, targets2, ignore_index, _DEFAULT_CHUNK if chunk_size is None else chunk_size)
     else:
-        nll, _, _ = kernel_forward_parts(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size,
-                                         mean=reduction == "mean")
+        nll = _kernel_loss(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size,
+                           mean=reduction == "mean")
         if reduction == "mean":
             return nll
     return _reduce(nll, reduction=reduction, leading=leading, targets2=targets2, ignore_index=ignore_index)

@@ -132,3 +132,138 @@ def test_packed_loss_kernel_path_runs_and_matches_reference_attention():
     m.config._mtp_flash_impl = "reference"
     lr, _ = make_packed_loss_fn(m, impl="naive")(m, *args)
     assert abs(lk.item() - lr.item()) < 2e-2 * abs(lr.item())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mask", ["causal", "full", "packed"])
+def test_attention_node_equals_the_python_function(dtype, mask):
+    """flash_attention's C++ node against the Python Function it stands for, bit for bit: strided inputs,
+    a strided and a missing output gradient, inputs without gradients, hooks on the saved tensors, two
+    backwards through one graph, evaluation, and the counters."""
+    from mlx_train_perf.attention import PackedMask, api, flash_attention
+
+    g = torch.Generator().manual_seed(5)
+
+    def strided(h):
+        return torch.randn(2, 130, h, 64, generator=g).to("cuda", dtype).transpose(1, 2)
+
+    q, do = strided(4), strided(4)
+    k, v = strided(2), strided(2)
+    seg = args = None
+    if mask == "packed":
+        sid = torch.tensor([[0] * 50 + [1] * 80] * 2)
+        sst = torch.tensor([[0] * 50 + [50] * 80] * 2)
+        seg = PackedMask(seg_id=sid.cuda(), seg_start=sst.cuda())
+        args = (seg.seg_id.int(), seg.seg_start.int())
+    leaves = [x.clone().detach().requires_grad_(True) for x in (q, k, v)]
+
+    def node(a, b, c):
+        return flash_attention(a, b, c, scale=0.125, causal=mask != "full", segments=seg)
+
+    def function(a, b, c):
+        return api._KernelAttention.apply(a.contiguous(), b.contiguous(), c.contiguous(), *(args or (None, None)), 0.125,
+                                          mask != "full")[0]
+
+    o, ref = node(*leaves), function(*leaves)
+    assert type(o.grad_fn) is not type(ref.grad_fn)
+    assert torch.equal(o, ref)
+    before = dict(api.VJP_CALLS)
+    want = torch.autograd.grad(ref, leaves, do)
+    got = torch.autograd.grad(o, leaves, do, retain_graph=True)
+    again = torch.autograd.grad(o, leaves, do)
+    assert all(torch.equal(a, w) and torch.equal(b, w) for a, b, w in zip(got, again, want))
+    assert all(api.VJP_CALLS[n] == before.get(n, 0) + 3 for n in ("flash_attention", "flash_attention_kernel_bwd"))
+    with pytest.raises(RuntimeError):   # freed by the second backward
+        torch.autograd.grad(o, leaves, do)
+    (dk,) = torch.autograd.grad(node(q, leaves[1], v), leaves[1], do)   # only k asks for a gradient
+    assert torch.equal(dk, want[1])
+    counts = []
+    for f in (node, function):
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+            out = f(*leaves)
+        assert all(torch.equal(a, w) for a, w in zip(torch.autograd.grad(out, leaves, do), want))
+        counts.append(sorted(packed))
+    assert counts[0] == counts[1]
+    with torch.no_grad():
+        assert torch.equal(node(q, k, v), o) and not node(q, k, v).requires_grad
+    with torch.inference_mode():
+        assert torch.equal(node(q, k, v), o)
+
+
+def test_attention_refuses_what_the_python_function_refuses():
+    """Function transforms and forward-mode gradients raise, as they do for the Python Function."""
+    from mlx_train_perf.attention import flash_attention
+
+    q = torch.randn(1, 2, 32, 64, device="cuda", dtype=torch.bfloat16)
+
+    def f(x):
+        return flash_attention(x, q, q, scale=0.125).float().sum()
+
+    with pytest.raises(RuntimeError):
+        torch.func.grad(f)(q)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(f)(q[None])
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):
+        f(torch.autograd.forward_ad.make_dual(q, q))
+
+
+LOSS_MODES = [{}, {"MTP_LCE_TRANSPOSED_HEAD": "0"}, {"MTP_LCE_TRANSPOSED_HEAD": "1"},
+              {"MTP_LCE_TRANSPOSED_HEAD": "0", "MTP_LCE_STAGE_HEAD": "0"}, {"MTP_LCE_BWD_BUDGET": "300000"}]
+
+
+@pytest.mark.parametrize("env", LOSS_MODES, ids=lambda e: ",".join(f"{k[8:]}={v}" for k, v in e.items()) or "default")
+@pytest.mark.parametrize(("kind", "dtype", "d"), [("frozen", torch.bfloat16, 128), ("frozen", torch.bfloat16, 72),
+                                                  ("trainable", torch.bfloat16, 128), ("q4", torch.bfloat16, 128),
+                                                  ("trainable", torch.float32, 36), ("q4", torch.float32, 64)])
+def test_loss_node_equals_the_python_function(kind, dtype, d, env, monkeypatch):
+    """linear_cross_entropy's C++ node against the Python Function it stands for, bit for bit, in every head
+    mode: both reductions, a strided gradient, an explicit chunk, hooks on the saved tensors, the counter,
+    two backwards, evaluation."""
+    from mlx_train_perf import DenseHead, QuantizedHead, _native, linear_cross_entropy
+    from mlx_train_perf.core import loss as L
+    from mlx_train_perf.core.quant import quantize
+
+    for name in ("MTP_LCE_TRANSPOSED_HEAD", "MTP_LCE_STAGE_HEAD", "MTP_LCE_BWD_BUDGET"):
+        monkeypatch.delenv(name, raising=False)
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    g = torch.Generator().manual_seed(9)
+    n, v = 321, 700
+    hidden = torch.randn(n, d, generator=g).to("cuda", dtype).requires_grad_(True)
+    w = (torch.randn(v, d, generator=g) * 0.05).to("cuda", dtype)
+    t = torch.randint(0, v, (n,), generator=g).cuda()
+    t[::7] = -100
+    wrt = [hidden]
+    if kind == "q4":
+        head = QuantizedHead(**dict(zip(("w_q", "scales", "biases"), quantize(w))))
+    else:
+        head = DenseHead(weight=w.requires_grad_(kind == "trainable"), trainable=kind == "trainable")
+        wrt += [w] if kind == "trainable" else []
+    ct = torch.rand(n, 2, generator=g).cuda()[:, 0]
+
+    def calls():
+        out = []
+        for kw in ({"reduction": "none"}, {"reduction": "mean"}, {"reduction": "none", "chunk_size": 256}):
+            loss = linear_cross_entropy(hidden, head, t, **kw)
+            grad = ct if kw["reduction"] == "none" else torch.tensor(0.5, device="cuda")
+            before = L.VJP_CALLS.get("kernel", 0)
+            first = torch.autograd.grad(loss, wrt, grad, retain_graph=True)
+            out += [loss.detach(), *first, *torch.autograd.grad(loss, wrt, grad)]
+            assert L.VJP_CALLS["kernel"] == before + 2
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: packed.append(x.shape) or x.cpu(), lambda x: x.cuda()):
+            loss = linear_cross_entropy(hidden, head, t)
+        out += torch.autograd.grad(loss, wrt)
+        with torch.no_grad():
+            out.append(linear_cross_entropy(hidden, head, t))
+            assert not out[-1].requires_grad
+        return out, sorted(packed), type(loss.grad_fn)
+
+    L.clear_transposed_head_cache()
+    got, packed, node = calls()
+    monkeypatch.setattr(_native, "plain", lambda *a: False)
+    want, packed_f, function = calls()
+    assert node is not function and packed == packed_f
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+    L.clear_transposed_head_cache()
