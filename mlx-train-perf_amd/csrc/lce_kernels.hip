@@ -1598,6 +1598,90 @@ void lce_bwd_dh_kernel(const bf16_t* __restrict__ G, int ldg, int kc, const bf16
 }
 
 
+// The same product for an output too small to fill the chip with 256 x 256 tiles: a workgroup owns 64 x 64
+// of dH, and its 8 waves contract an eighth of the vocab each, fragments straight from memory (64 bytes of
+// a row per lane and 64-deep slab; the operands are read once per 64 columns or rows of the other, out
+// of the caches at these sizes), one slab ahead. The 8 fp32 tiles are summed through LDS in wave order. One
+// output tile of the kernel above is a chain of 64-deep stages on one CU, latency bound at about
+// 1.3 us a stage: N = 128, D = 256, V = 3000 (48 stages) 64 us, here 23. The loads' latency bounds this one
+// too: a slab of a wave is 128 rows' lines, more than the CU's L1 holds for 8 waves.
+// Wt is required (both operands K-contiguous) and D % 64 == 0; mode as above.
+constexpr int kSmallTile = 64;
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void lce_bwd_dh_small_kernel(const bf16_t* __restrict__ G, int ldg, int kc, const bf16_t* __restrict__ Wt, int ldt,
+                             int tcol0, int N, int D, float* __restrict__ acc32, bf16_t* __restrict__ dH, int mode) {
+  __shared__ __attribute__((aligned(16))) float part[8][kSmallTile][kSmallTile];
+  const int dtiles = D / kSmallTile;
+  const int t0 = (blockIdx.x / dtiles) * kSmallTile, d0 = (blockIdx.x % dtiles) * kSmallTile;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, i = lane & 31;
+  const int nb = kc / kBK, b0 = w * nb / 8, b1 = (w + 1) * nb / 8;
+  const bf16_t* ga[2];
+  const bf16_t* wb[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int t = t0 + 32 * x + i;
+    ga[x] = G + (long)(t < N ? t : N - 1) * ldg + 32 * h;
+    wb[x] = Wt + (long)(d0 + 32 * x + i) * ldt + tcol0 + 32 * h;
+  }
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.f;
+  // Lane half h contracts k 32 h .. 32 h + 31 of a slab, 8 at a step, in both operands.
+  u32x4 fa[2][2][4], fb[2][2][4];
+  auto load = [&](int b, u32x4 (&a)[2][4], u32x4 (&c)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        a[x][s] = *reinterpret_cast<const u32x4*>(ga[x] + (long)b * kBK + 8 * s);
+        c[x][s] = *reinterpret_cast<const u32x4*>(wb[x] + (long)b * kBK + 8 * s);
+      }
+  };
+  auto product = [&](const u32x4 (&a)[2][4], const u32x4 (&c)[2][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = mfma32(as_bf16x8(a[x][s]), as_bf16x8(c[y][s]), acc[x][y]);
+  };
+  if (b0 < b1) load(b0, fa[0], fb[0]);
+  for (int b = b0; b < b1; b += 2) {
+    if (b + 1 < b1) load(b + 1, fa[1], fb[1]);
+    product(fa[0], fb[0]);
+    if (b + 2 < b1) load(b + 2, fa[0], fb[0]);
+    if (b + 1 < b1) product(fa[1], fb[1]);
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) part[w][32 * x + 8 * (r >> 2) + 4 * h + (r & 3)][32 * y + i] = acc[x][y][r];
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int e = threadIdx.x + kThreads * p, row = e >> 4, col = 4 * (e & 15), t = t0 + row;
+    f32x4 s = *reinterpret_cast<const f32x4*>(&part[0][row][col]);
+#pragma unroll
+    for (int q = 1; q < 8; ++q) s += *reinterpret_cast<const f32x4*>(&part[q][row][col]);
+    if (t >= N) continue;
+    const long o = (long)t * D + d0 + col;
+    if (mode == 0) {
+      *reinterpret_cast<f32x4*>(acc32 + o) = s;
+    } else if (mode == 1) {
+      *reinterpret_cast<f32x4*>(acc32 + o) += s;
+    } else {
+      if (mode == 2) s += *reinterpret_cast<const f32x4*>(acc32 + o);
+      *reinterpret_cast<u32x2*>(dH + o) = u32x2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+    }
+  }
+}
+
 // Sum of a split dH product's fp32 parts (in part order, so the result does not depend on which
 // workgroup finished first), then the mode of lce_bwd_dh_kernel. One block per 4 rows of a tile,
 // one thread per 4 columns (D % 4 == 0, so a group of 4 is inside or past D as a whole).
@@ -1862,6 +1946,16 @@ size_t lce_dh_parts_bytes(long rows, long D, long ktiles) {
   return (size_t)ks * (size_t)tiles * kTile * kTile * sizeof(float);
 }
 
+// Whether a dH product over `ktiles` vocab tiles, in `ks` parts of 256 x 256 tiles otherwise, takes the
+// 64 x 64 tiles of lce_bwd_dh_small_kernel: at most two rounds of its workgroups, and a vocab too short to
+// be split (from 16 tiles on the large tiles' parts are faster). Whole backward, large against small
+// tiles, N x D x V: 128 x 256 x 3000 80 / 39 us, 1024 x 1024 x 3000 99 / 56, 512 x 2048 x 3000 115 / 72,
+// 2048 x 1024 x 3000 (512 workgroups) 101 / 79; beyond: 1024 x 4096 x 3000 (1024) 148 / 171,
+// 1024 x 1024 x 10000 (40 vocab tiles) 82 / 107.
+static bool lce_dh_small(long rows, long D, long ktiles, int ks) {
+  return ks == 1 && ktiles < 16 && (rows + kSmallTile - 1) / kSmallTile * (D / kSmallTile) <= 2 * kNumCU;
+}
+
 // Block edge for xcd_split_tile: the sa x (32 / sa) block with the fewest panels per stage that
 // divides the tile grid, or 0 (row-major order) when none does.
 static int lce_dh_split_a(int rtiles, int dtiles) {
@@ -2094,26 +2188,34 @@ static hipError_t lce_bwd_rows(const LceHead& h, const bf16_t* H, const int64_t*
     else if (c == nchunks - 1) mode = 2;
     else mode = 1;
     const int ks = lce_dh_ksplit(N, D, ctiles);
-    const int sa = ks > 1 ? lce_dh_split_a(rtiles, dtiles) : 0;
-    dim3 hgrid(8 * rtiles * ((dtiles + 7) / 8));
-    if (ks > 1) {
-      const int blocks = sa ? (rtiles / sa) * (dtiles / (32 / sa)) * ks : 0;
-      hgrid = dim3(sa ? (blocks + 7) / 8 * 256 : rtiles * dtiles * ks);
-    }
-    if (h.q4) {
-      hipLaunchKernelGGL(lce_bwd_dh_kernel<1>, hgrid, block, 0, stream, Gbuf, ldg, ctiles * kTile, h.w, wt, ldw,
-                         tcol0, h.wq, h.sc, h.bi, N, D, V, vb, ve, acc32, dH, mode, ks, sa, parts);
-    } else {
-      hipLaunchKernelGGL(lce_bwd_dh_kernel<0>, hgrid, block, 0, stream, Gbuf, ldg, ctiles * kTile, h.w, wt, ldw,
-                         tcol0, h.wq, h.sc, h.bi, N, D, V, vb, ve, acc32, dH, mode, ks, sa, parts);
-    }
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (ks > 1) {
-      hipLaunchKernelGGL(lce_bwd_dh_reduce_kernel, dim3(rtiles * dtiles * 64), dim3(256), 0, stream, parts, ks, N, D,
+    if (wt != nullptr && D % kBK == 0 && lce_dh_small(N, D, ctiles, ks)) {
+      const int wgs = (N + kSmallTile - 1) / kSmallTile * (D / kSmallTile);
+      hipLaunchKernelGGL(lce_bwd_dh_small_kernel, dim3(wgs), block, 0, stream, Gbuf, ldg, ctiles * kTile, wt, ldw, tcol0, N, D,
                          acc32, dH, mode);
       e = hipGetLastError();
       if (e != hipSuccess) return e;
+    } else {
+      const int sa = ks > 1 ? lce_dh_split_a(rtiles, dtiles) : 0;
+      dim3 hgrid(8 * rtiles * ((dtiles + 7) / 8));
+      if (ks > 1) {
+        const int blocks = sa ? (rtiles / sa) * (dtiles / (32 / sa)) * ks : 0;
+        hgrid = dim3(sa ? (blocks + 7) / 8 * 256 : rtiles * dtiles * ks);
+      }
+      if (h.q4) {
+        hipLaunchKernelGGL(lce_bwd_dh_kernel<1>, hgrid, block, 0, stream, Gbuf, ldg, ctiles * kTile, h.w, wt, ldw,
+                           tcol0, h.wq, h.sc, h.bi, N, D, V, vb, ve, acc32, dH, mode, ks, sa, parts);
+      } else {
+        hipLaunchKernelGGL(lce_bwd_dh_kernel<0>, hgrid, block, 0, stream, Gbuf, ldg, ctiles * kTile, h.w, wt, ldw,
+                           tcol0, h.wq, h.sc, h.bi, N, D, V, vb, ve, acc32, dH, mode, ks, sa, parts);
+      }
+      e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      if (ks > 1) {
+        hipLaunchKernelGGL(lce_bwd_dh_reduce_kernel, dim3(rtiles * dtiles * 64), dim3(256), 0, stream, parts, ks, N, D,
+                           acc32, dH, mode);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+      }
     }
     if (dW != nullptr && !h.q4) {
       dim3 wgrid(8 * ctiles * ((dtiles + 7) / 8));

@@ -469,6 +469,33 @@ def test_backward_split_contraction(n, d, v, head, with_wt):
 
 # (n, d, v, chunk, head): one chunk and several (the last one partial), a split dH contraction
 # (n = 1000, d = 2048), a tiny grid and a 256-column chunk; 4-bit and dense heads.
+# The 64 x 64-tile dH product (a vocabulary of up to 15 tiles): row counts around its tiles and its 512
+# workgroups, one to three slabs per wave, several chunks (its fp32 accumulator), and the first sizes past it.
+@pytest.mark.parametrize(("n", "d", "v", "chunk"), [(1, 64, 1, None), (64, 128, 256, None), (65, 192, 1000, 256),
+                                                    (200, 64, 3840, None), (130, 320, 3841, None), (257, 256, 1100, 512),
+                                                    (1024, 2048, 500, None), (1025, 2048, 500, None)])
+@pytest.mark.parametrize("head", ["frozen", "trainable", "q4"])
+def test_backward_small_output_tiles(n, d, v, chunk, head):
+    from mlx_train_perf.core.loss import DenseHead, QuantizedHead, kernel_forward_parts
+
+    h, w, t = lce_inputs(n, d, v, seed=n + d + v)
+    hd = h.cuda().requires_grad_(True)
+    if head == "q4":
+        wq, sc, bi = oquant.quantize_affine(w.float())
+        w = oquant.dequantize_affine(wq, sc, bi, dtype=torch.float32).to(torch.bfloat16)
+        kh = QuantizedHead(w_q=wq.cuda(), scales=sc.cuda(), biases=bi.cuda())
+    else:
+        kh = DenseHead(weight=w.cuda().requires_grad_(head == "trainable"), trainable=head == "trainable")
+    nll, _, _ = kernel_forward_parts(hd, kh, t.cuda(), ignore_index=IGN, bwd_chunk=chunk)
+    ct = _cotangent(t)
+    nll.backward(ct.cuda())
+    _, olse, _ = olce.forward(h.cuda(), w.cuda(), t.cuda(), ignore_index=IGN)
+    odh = olce.backward(h.cuda(), w.cuda(), t.cuda(), olse, ct.cuda(), ignore_index=IGN, dtype=torch.float64)
+    assert torch.isfinite(hd.grad).all()
+    # a vocabulary of one class has no gradient but its rounding
+    assert rel_l2(hd.grad.cpu(), odh.cpu()) <= 1e-2 or (v == 1 and float(hd.grad.float().norm()) < 1e-3)
+
+
 @pytest.mark.parametrize(("n", "d", "v", "chunk", "head"), [(1000, 512, 6000, 2048, "q4"),
                                                             (1000, 2048, 8000, 8192, "q4"),
                                                             (300, 256, 3000, 256, "q4"),
