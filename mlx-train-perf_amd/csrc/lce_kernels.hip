@@ -1278,13 +1278,19 @@ void lce_bwd_g_kernel(const bf16_t* __restrict__ H, const bf16_t* __restrict__ W
 // wrow0 + r (0 for the whole head, the chunk's first row for dequantized rows staged per chunk).
 // Workgroup (row tile, vocab split) walks its split's vocab tiles of the chunk back to back on the
 // DMA core, in the forward's XCD-grouped order; the next tile's first two stages are issued during the current
-// tile's last k-step. Each lane stores its G values straight from the accumulator layout (8-byte
-// buffer stores of 4 columns; the write-back L2 merges a row's 16 segments into whole lines), so
-// the epilogue needs no barrier and its stores drain while the next tile's MFMAs run: every
-// thread issues exactly kGStores stores per tile and the next tile's first wait leaves those in
-// flight.
+// tile's last k-step. Each wave turns its G values through LDS of its own, in blocks of 32 tokens x 64
+// columns, and stores them 16 bytes per lane, whole 128-byte lines: the epilogue needs no barrier and
+// its stores drain while the next tile's MFMAs run (every thread issues exactly kGStores stores per
+// tile and the next tile's first wait leaves those in flight).
+// A dense head's tile is bound by its product, then by this epilogue, the more the fewer k-stages a tile has;
+// 8-byte stores straight from the accumulator layout wrote each line in 16 pieces. Backward alone, before and
+// after, N x D x V: 8192 x 4096 x 128256 13.01 -> 12.76 ms, 4096 x 1536 x 100000 2226 -> 2098 us,
+// 2048 x 896 x 151936 1133 -> 1055 us, 8192 x 1024 x 50000 1541 -> 1418 us.
+// The blocks lie past the two stages (dense head: 160 KB in all), or in the first stage's head tile, which the
+// 4-bit head's next tile fills only after its first barrier.
 // ------------------------------------------------------------------------------------------
-constexpr int kGStores = 4 * 4 * kNJ;
+constexpr int kGBlockBytes = 4096;   // a wave's staging block: 32 tokens x 64 columns
+constexpr int kGStores = 2 * 4 * kNJ;  // 16-byte stores per thread and tile
 
 template <int Q4>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -1294,7 +1300,9 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
                               const float* __restrict__ lse, const float* __restrict__ dnll, long long ignore_index,
                               int N, int D, int V, int v_begin, int v_end, int ctiles, int nsplit, int ldg,
                               int wrow0, bf16_t* __restrict__ G) {
-  __shared__ __attribute__((aligned(16))) char lds[Q4 ? kLdsBytes + kQ4SbBytes : kLdsBytes];
+  // One array: with a second one the compiler tracks the copies into LDS by array and waits for all
+  // of them (vmcnt(0)) before fragment reads of every stage (flagship 4.09 -> 4.62 ms).
+  __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes + (Q4 ? kQ4SbBytes : 8 * kGBlockBytes)];
 
   const int g = blockIdx.x;
   const int rtiles = (N + kTile - 1) / kTile;
@@ -1319,19 +1327,15 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
   const int t0 = rt * kTile;
   const int nk = D / kBK;
   const int vlim = v_end < V ? v_end : V;
-  const int colb = 128 * wa + 4 * lhalf;  // this lane's first G column within a tile
 
-  // Per-thread token rows (fixed for the workgroup): coefficient, log2-domain lse and the row's G
-  // byte offset.
+  // Per-thread token rows (fixed for the workgroup): coefficient and log2-domain lse.
   float coef[kNJ], l2[kNJ];
-  uint32_t gvo[kNJ];
 #pragma unroll
   for (int j = 0; j < kNJ; ++j) {
     const int r = 64 * wb + 32 * j + lcol;
     const int t = t0 + r;
     coef[j] = 0.f;
     l2[j] = 0.f;
-    gvo[j] = 2u * (uint32_t)(r * ldg + colb);
     if (t < N) {
       coef[j] = targets[t] == ignore_index ? 0.f : dnll[t];
       l2[j] = lse[t] * kLog2e;
@@ -1340,6 +1344,11 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
   // G rows of this row tile; stores to rows past N fall outside the range and are dropped.
   const int grows = N - t0 < kTile ? N - t0 : kTile;
   const __amdgpu_buffer_rsrc_t gr = dma_rsrc(reinterpret_cast<const char*>(G + (long)t0 * ldg), 2L * grows * ldg);
+
+  // Staged stores: this wave's block, and the lane's byte offset in G (row 64 wb + lane / 8, 16 bytes of the
+  // wave's first 64 columns).
+  char* gst = lds + (Q4 ? 0 : kLdsBytes) + w * kGBlockBytes;
+  const uint32_t gso = 2u * (uint32_t)((64 * wb + (lane >> 3)) * ldg + 128 * wa + 8 * (lane & 7));
 
   DmaRowOp ob;
   ob.init(H + (long)t0 * D, D, N - t0);
@@ -1402,20 +1411,42 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
     // each row's target column and the zeros of the columns past the chunk's last vocab row (the
     // chunk's last tile only; their head rows are clamped copies of a valid row, so these values
     // are finite) are written afterwards by lce_bwd_g_fix_kernel. Tile column of acc[i][j][4q + u]
-    // is colb + 32 i + 8 q + u.
+    // is 128 wa + 32 i + 8 q + 4 lhalf + u.
     const int tl = v0 - v_begin;
+    auto value = [&](int i, int j, int q) __attribute__((always_inline)) {
+      float gv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) gv[u] = fast_exp2(acc[i][j][4 * q + u] * kLog2e - l2[j]) * coef[j];
+      return u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
+    };
+    // Blocks of 32 tokens x 64 columns through the wave's staging block ([token][128 B], 16-byte chunk c
+    // at slot c ^ (token / 2) % 8), so that a store writes whole 128-byte lines of 8 rows. DS operations
+    // of a wave run in order, so a block's writes follow the reads of the one before. The lane's bases
+    // pass through an empty asm, so that the 16 offsets of the stores and the 12 in LDS are formed here
+    // instead of being held in registers over the product.
+    uint32_t go = gso, wo = (uint32_t)(lcol * 128 + (((lcol >> 1) & 7) << 4) + 8 * lhalf),
+             ro = (uint32_t)((lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 4) & 7)) << 4));
+    asm volatile("" : "+v"(go), "+v"(wo), "+v"(ro));
 #pragma unroll
     for (int j = 0; j < kNJ; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int ip = 0; ip < 2; ++ip) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float gv[4];
+        for (int c = 0; c < 8; ++c)
+          *reinterpret_cast<u32x2*>(gst + (wo ^ (c << 4))) = value(2 * ip + (c >> 2), j, c & 3);
+        u32x4 x[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) gv[u] = fast_exp2(acc[i][j][4 * q + u] * kLog2e - l2[j]) * coef[j];
-          const u32x2 val = u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
-          __builtin_amdgcn_raw_buffer_store_b64(val, gr, gvo[j] + 64 * i + 16 * q, 2 * tl, 0);
-        }
+        for (int p = 0; p < 4; ++p)  // row 8 p + lane / 8: (row / 2) % 8 = 4 (p % 2) + lane / 16
+          x[p] = *reinterpret_cast<const u32x4*>(gst + (ro ^ ((p & 1) << 6)) + 1024 * p);
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          __builtin_amdgcn_raw_buffer_store_b128(x[p], gr, go + (uint32_t)((32 * j + 8 * p) * 2 * ldg + 128 * ip), 2 * tl, 0);
+        // The data registers stay as they are for some cycles: a store of 16 bytes per lane reads them
+        // after it has issued, lanes 12-15 of each 16 last. With an SGPR offset the compiler takes the
+        // store to need no wait before a VALU write to them, and v_add right after one put an address
+        // into the first dword of exactly those lanes of G (seen, not always, on gfx950).
+        asm volatile("s_nop 7" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+      }
   }
 }
 

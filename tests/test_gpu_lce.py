@@ -467,6 +467,28 @@ def test_backward_split_contraction(n, d, v, head, with_wt):
     assert (outs[0][t == IGN] == 0).all()
 
 
+# G tiles stored a line at a time from LDS by workgroups that walk several vocab tiles: one to four k-stages,
+# even and odd; whole and ragged row tiles; a last vocab tile of one column; both heads. A row's bound is that
+# of its bf16 result (2^-8) and of G entries whose fp32 exponential falls on the other side of a bf16 rounding
+# (under 2^-8 of the entry, few of a row); an entry replaced by other bits exceeds it.
+@pytest.mark.parametrize(("n", "d", "v"), [(2048, 64, 33025), (1000, 128, 70000), (257, 192, 140000), (2048, 256, 40000)])
+@pytest.mark.parametrize("head", ["dense", "q4"])
+def test_backward_many_vocab_tiles_per_workgroup(n, d, v, head):
+    print(f"[lce bwd many tiles] n={n} d={d} v={v} head={head}", flush=True)
+    assert (n + 255) // 256 * ((v + 255) // 256) > 2 * 256
+    h, w, t = lce_inputs(n, d, v, seed=n + d + v, w_std=0.05)
+    t[::3] = IGN
+    ct = _cotangent(t)
+    outs, wf = _capi_backward(h, w, t, ct, head=head, with_wt=True, reps=3)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert (outs[0][t == IGN] == 0).all()
+    h, wf, t, ct = h.cuda(), wf.to(torch.bfloat16).cuda(), t.cuda(), ct.cuda()  # a 4-bit head's products take bf16 weights
+    _, olse, _ = olce.forward(h, wf, t, ignore_index=IGN)
+    odh = olce.backward(h, wf, t, olse, ct, ignore_index=IGN, round_g_bf16=True, dtype=torch.float64).cpu()
+    row = (outs[0].double() - odh).norm(dim=1) / odh.norm(dim=1).clamp_min(1e-30)
+    assert row.max() <= 2.0 ** -7
+
+
 # (n, d, v, chunk, head): one chunk and several (the last one partial), a split dH contraction
 # (n = 1000, d = 2048), a tiny grid and a 256-column chunk; 4-bit and dense heads.
 # The 64 x 64-tile dH product (a vocabulary of up to 15 tiles): row counts around its tiles and its 512
