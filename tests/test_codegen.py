@@ -3,11 +3,11 @@ objects `build()` leaves in `mlx-train-perf_amd/_build/` (the device code object
 from its fat binary).
 
 1. Wide stores: a 12- or 16-byte store's data registers written by either of the next two
-   instructions with no `s_nop` between. Reverted gradient-tile variants with 16-byte stores had
-   this pattern and gave intermittently wrong rows. It is a guard, not an explanation: the
-   documented gfx9 rule (LLVM's GCNHazardRecognizer::createsVALUHazard) asks for that wait state
-   only when the store's soffset is not a register, and those stores took an SGPR soffset, so this
-   pair is probably not what went wrong.
+   instructions with no `s_nop` between. Gradient-tile variants with 16-byte stores that had this
+   pattern gave wrong rows now and then: the wrong entries were those of the store that such a write
+   followed, and held what it wrote. The documented gfx9 rule (LLVM's
+   GCNHazardRecognizer::createsVALUHazard) asks for that wait state only when the store's soffset
+   is not a register, and those stores took an SGPR soffset, so the compiler leaves none.
 2. Lane swaps: a `v_permlane{16,32}_swap` whose operands a VALU op writes within 2 wait states
    (or whose exec a `v_cmpx` writes within 4), the gfx950 hazard the reverted variant's swaps also
    came close to. The shipped kernels' swaps are inline asm with `s_nop 1` before them."""
