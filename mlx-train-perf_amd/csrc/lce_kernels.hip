@@ -1273,6 +1273,50 @@ void lce_bwd_g_kernel(const bf16_t* __restrict__ H, const bf16_t* __restrict__ W
 }
 
 // ------------------------------------------------------------------------------------------
+// A wave's sub-tile (128 A x 64 B of gemm_dma) to bf16 rows of B's index, 16 bytes per lane: blocks of
+// 32 rows x 64 columns go through the wave's block of LDS ([row][128 B], 16-byte chunk c at slot
+// c ^ (row / 2) % 8), so that a store writes whole 128-byte lines of 8 rows. value(i, j, q) packs the four
+// columns 32 i + 8 q + 4 (lane / 32) + 0..3 of row 32 j + lane % 32; offset(ip) is the byte offset of row
+// lane / 8, columns 64 ip + 8 (lane % 8) .. + 7, of the sub-tile. DS operations of a wave run in order, so a
+// block's writes follow the reads of the one before. kGStores stores per thread.
+// ------------------------------------------------------------------------------------------
+constexpr int kGBlockBytes = 4096;   // a wave's staging block: 32 tokens x 64 columns
+constexpr int kGStores = 2 * 4 * kNJ;  // 16-byte stores per thread and tile
+
+
+__device__ __forceinline__ void store16(const u32x4& x, const __amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(x, r, voff, soff, 0);
+}
+template <class VAL, class OFF>
+__device__ __forceinline__ void store_lines(char* blk, const __amdgpu_buffer_rsrc_t r, int ld, int soff,
+                                            const VAL& value, const OFF& offset) {
+  const int lane = threadIdx.x & 63, row = lane & 31;
+  // Through an empty asm: the LDS offsets are formed here instead of being held over the product.
+  uint32_t wo = (uint32_t)(row * 128 + (((row >> 1) & 7) << 4) + 8 * (lane >> 5)),
+           ro = (uint32_t)((lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 4) & 7)) << 4));
+  asm volatile("" : "+v"(wo), "+v"(ro));
+#pragma unroll
+  for (int j = 0; j < kNJ; ++j)
+#pragma unroll
+    for (int ip = 0; ip < 2; ++ip) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        *reinterpret_cast<u32x2*>(blk + (wo ^ (c << 4))) = value(2 * ip + (c >> 2), j, c & 3);
+      u32x4 x[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p)  // row 8 p + lane / 8: (row / 2) % 8 = 4 (p % 2) + lane / 16
+        x[p] = *reinterpret_cast<const u32x4*>(blk + (ro ^ ((p & 1) << 6)) + 1024 * p);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) store16(x[p], r, offset(ip) + (uint32_t)((32 * j + 8 * p) * 2 * ld), soff);
+      // The data registers stay as they are for some cycles: a store of 16 bytes per lane reads them
+      // after it has issued, lanes 12-15 of each 16 last. With an SGPR offset the compiler takes the
+      // store to need no wait before a VALU write to them, and v_add right after one put an address
+      // into the first dword of exactly those lanes of G (seen, not always, on gfx950).
+      asm volatile("s_nop 7" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // Backward step 1, persistent form (hidden dim a multiple of 64), without the one-hot term and
 // the zero padding columns (see lce_bwd_g_fix_kernel). Row r of the dense W holds vocab row
 // wrow0 + r (0 for the whole head, the chunk's first row for dequantized rows staged per chunk).
@@ -1289,9 +1333,6 @@ void lce_bwd_g_kernel(const bf16_t* __restrict__ H, const bf16_t* __restrict__ W
 // The blocks lie past the two stages (dense head: 160 KB in all), or in the first stage's head tile, which the
 // 4-bit head's next tile fills only after its first barrier.
 // ------------------------------------------------------------------------------------------
-constexpr int kGBlockBytes = 4096;   // a wave's staging block: 32 tokens x 64 columns
-constexpr int kGStores = 2 * 4 * kNJ;  // 16-byte stores per thread and tile
-
 template <int Q4>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __restrict__ W,
@@ -1323,7 +1364,7 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6;
   const int wa = w & 1, wb = w >> 1;
-  const int lhalf = lane >> 5, lcol = lane & 31;
+  const int lcol = lane & 31;
   const int t0 = rt * kTile;
   const int nk = D / kBK;
   const int vlim = v_end < V ? v_end : V;
@@ -1411,7 +1452,7 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
     // each row's target column and the zeros of the columns past the chunk's last vocab row (the
     // chunk's last tile only; their head rows are clamped copies of a valid row, so these values
     // are finite) are written afterwards by lce_bwd_g_fix_kernel. Tile column of acc[i][j][4q + u]
-    // is 128 wa + 32 i + 8 q + 4 lhalf + u.
+    // is 128 wa + 32 i + 8 q + 4 (lane / 32) + u.
     const int tl = v0 - v_begin;
     auto value = [&](int i, int j, int q) __attribute__((always_inline)) {
       float gv[4];
@@ -1419,34 +1460,9 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
       for (int u = 0; u < 4; ++u) gv[u] = fast_exp2(acc[i][j][4 * q + u] * kLog2e - l2[j]) * coef[j];
       return u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
     };
-    // Blocks of 32 tokens x 64 columns through the wave's staging block ([token][128 B], 16-byte chunk c
-    // at slot c ^ (token / 2) % 8), so that a store writes whole 128-byte lines of 8 rows. DS operations
-    // of a wave run in order, so a block's writes follow the reads of the one before. The lane's bases
-    // pass through an empty asm, so that the 16 offsets of the stores and the 12 in LDS are formed here
-    // instead of being held in registers over the product.
-    uint32_t go = gso, wo = (uint32_t)(lcol * 128 + (((lcol >> 1) & 7) << 4) + 8 * lhalf),
-             ro = (uint32_t)((lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 4) & 7)) << 4));
-    asm volatile("" : "+v"(go), "+v"(wo), "+v"(ro));
-#pragma unroll
-    for (int j = 0; j < kNJ; ++j)
-#pragma unroll
-      for (int ip = 0; ip < 2; ++ip) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          *reinterpret_cast<u32x2*>(gst + (wo ^ (c << 4))) = value(2 * ip + (c >> 2), j, c & 3);
-        u32x4 x[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p)  // row 8 p + lane / 8: (row / 2) % 8 = 4 (p % 2) + lane / 16
-          x[p] = *reinterpret_cast<const u32x4*>(gst + (ro ^ ((p & 1) << 6)) + 1024 * p);
-#pragma unroll
-        for (int p = 0; p < 4; ++p)
-          __builtin_amdgcn_raw_buffer_store_b128(x[p], gr, go + (uint32_t)((32 * j + 8 * p) * 2 * ldg + 128 * ip), 2 * tl, 0);
-        // The data registers stay as they are for some cycles: a store of 16 bytes per lane reads them
-        // after it has issued, lanes 12-15 of each 16 last. With an SGPR offset the compiler takes the
-        // store to need no wait before a VALU write to them, and v_add right after one put an address
-        // into the first dword of exactly those lanes of G (seen, not always, on gfx950).
-        asm volatile("s_nop 7" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
-      }
+    uint32_t go = gso;
+    asm volatile("" : "+v"(go));  // the 16 offsets of the stores are formed here, not held over the product
+    store_lines(gst, gr, ldg, 2 * tl, value, [&](int ip) { return go + 128 * ip; });
   }
 }
 
@@ -1746,6 +1762,9 @@ __global__ __launch_bounds__(256) void lce_bwd_dh_reduce_kernel(const float* __r
 // Any N and any D that is a multiple of 8: token rows past N read as zeros and columns past D are not
 // stored. (Token counts are rarely multiples of 64, a trainer drops one position of each row; they took a
 // register-staged core that spilled: 1918 us against 954 at N = 8188, D = 2048, V = 32000, 1125 TFLOP/s.)
+// Bound by the products' LDS reads; the store of a tile stands alone (one workgroup per CU, one tile each), so
+// it counts the more the fewer the tokens: whole lines instead of 2 bytes per lane took this kernel from 404 to
+// 347 us at 512 x 2048 x 128000 and 146 to 130 at 1023 x 1024 x 32000 (8188 tokens: within noise).
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void lce_bwd_dw_kernel(const bf16_t* __restrict__ G, int ldg, const bf16_t* __restrict__ H, int N, int D, int V,
@@ -1757,33 +1776,32 @@ void lce_bwd_dw_kernel(const bf16_t* __restrict__ G, int ldg, const bf16_t* __re
   const int tid = threadIdx.x;
   const int lane = tid & 63, w = tid >> 6;
   const int wa = w & 1, wb = w >> 1;
-  const int lhalf = lane >> 5, lcol = lane & 31;
   const int vlim = v_end < V ? v_end : V;
   const int v0 = v_begin + vt * kTile;
   const int d0 = dt * kTile;
   const int nk = (N + kBK - 1) / kBK;
 
   f32x16 acc[4][kNJ];
-  // The vocab tile lies inside the chunk buffer (ctiles * 256 <= ldg), so all 256 G columns
-  // are readable; rows past the chunk's end are not stored below.
+  // H is A, so that a lane of the result holds runs of dims of one vocab row. The vocab tile lies inside the
+  // chunk buffer (ctiles * 256 <= ldg), so all 256 G columns are readable; rows past the chunk's end are
+  // not stored below.
   DmaTransOp oa;
-  oa.init(G + (v0 - v_begin), ldg, N, kTile);
+  oa.init(H + d0, D, N, D - d0);
   DmaTransOp ob;
-  ob.init(H + d0, D, N, D - d0);
+  ob.init(G + (v0 - v_begin), ldg, N, kTile);
   gemm_dma(oa, ob, nk, lds, acc, false, false, NoNext{});
 
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int v = v0 + 128 * wa + 32 * i + 8 * (r >> 2) + 4 * lhalf + (r & 3);
-      if (v >= vlim) continue;
-#pragma unroll
-      for (int j = 0; j < kNJ; ++j) {
-        const int d = d0 + 64 * wb + 32 * j + lcol;
-        if (d < D) dW[(long)v * D + d] = __builtin_bit_cast(bf16_t, (__bf16)acc[i][j][r]);
-      }
-    }
+  // Past the last barrier no wave reads or copies into the stages. Rows past the chunk's end lie past the
+  // descriptor's range, chunks past D (a multiple of 8) get an offset past it.
+  const __amdgpu_buffer_rsrc_t wr =
+      dma_rsrc(reinterpret_cast<const char*>(dW + (long)v0 * D), 2L * (vlim - v0 < kTile ? vlim - v0 : kTile) * D);
+  const int d = d0 + 128 * wa + 8 * (lane & 7);
+  const uint32_t row = 2u * (uint32_t)((64 * wb + (lane >> 3)) * D + d);
+  auto value = [&](int i, int j, int q) __attribute__((always_inline)) {
+    return u32x2{pack_bf16x2(acc[i][j][4 * q], acc[i][j][4 * q + 1]), pack_bf16x2(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
+  };
+  store_lines(lds + w * kGBlockBytes, wr, D, 0, value,
+              [&](int ip) { return d + 64 * ip < D ? row + 128 * ip : 0x7ffffff0u; });
 }
 
 // ------------------------------------------------------------------------------------------

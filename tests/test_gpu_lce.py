@@ -192,7 +192,7 @@ def test_trainable_head_dw_parity(n, d, v, chunk):
 # Token counts around the 64-deep stages of the dW product and hidden dims around its 256-column tiles,
 # several chunks and a vocabulary that ends inside a tile.
 @pytest.mark.parametrize(("n", "d", "v", "chunk"), [(1, 64, 300, 256), (63, 72, 300, None), (65, 256, 700, 256),
-                                                    (127, 264, 513, None), (257, 200, 300, 256), (447, 320, 300, None)])
+                                                    (127, 264, 513, None), (257, 200, 300, 256), (447, 320, 300, None), (130, 328, 900, 512)])
 def test_trainable_head_dw_ragged_tokens(n, d, v, chunk):
     test_trainable_head_dw_parity(n, d, v, chunk)
 
