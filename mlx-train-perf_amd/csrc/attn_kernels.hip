@@ -1016,19 +1016,44 @@ void attn_kv_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, 
     lt = l + __shfl_xor(l, 32, 64);
     mul = (lt > 0.f) ? 1.f / lt : 0.f;
   }
-  if (qvalid) {
+  if constexpr (!DQ) {
+    if (qvalid && hf == 0) lse_out[qrow + qi] = (m + fast_log2(lt)) * kLn2;
+  }
+  auto quad = [&](int db, int rq) __attribute__((always_inline)) {  // dims 32 db + 8 rq + 4 hf .. + 3
+    return u32x2{pack_bf16x2(acc[db][4 * rq] * mul, acc[db][4 * rq + 1] * mul),
+                 pack_bf16x2(acc[db][4 * rq + 2] * mul, acc[db][4 * rq + 3] * mul)};
+  };
+  if constexpr (DH == 96) {
+    // Rows of 192 bytes, a line and a half: through LDS measured the same (88.8 and 89.0 us at
+    // 2 x 16/4 x 2050, not causal).
+    if (!qvalid) return;
     bf16_t* oh = out + (qrow + qi) * DH;
-    if constexpr (!DQ) {
-      if (hf == 0) lse_out[qrow + qi] = (m + fast_log2(lt)) * kLn2;
-    }
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int d = 32 * db + 8 * rq + 4 * hf;
-        *reinterpret_cast<u32x2*>(oh + d) = u32x2{pack_bf16x2(acc[db][4 * rq] * mul, acc[db][4 * rq + 1] * mul),
-                                                  pack_bf16x2(acc[db][4 * rq + 2] * mul, acc[db][4 * rq + 3] * mul)};
-      }
+      for (int rq = 0; rq < 4; ++rq) *reinterpret_cast<u32x2*>(oh + 32 * db + 8 * rq + 4 * hf) = quad(db, rq);
+  } else {
+    if (!wave_has) return;
+    // The wave's 32 rows through its quarter of stage 0 (nobody reads or copies into it past the last
+    // barrier), so that a store writes whole rows: 16-byte chunk c of row r at slot c ^ r (head_dim 64:
+    // c ^ r / 2) of its 256 (128) bytes. 8 bytes per lane from the accumulator layout wrote a line in 16
+    // pieces, which counts where walks are short: packed S = 16384 (~12 key tiles a walk) forward 261 -> 252
+    // us and backward 806 -> 792, 4 x 16/4 x 1000 x 128 causal 29.3 -> 27.2 and 100.2 -> 97.8, S = 8192
+    // causal 497 -> 492 and 1617 -> 1614.
+    char* ob = lds0 + w * (32 * kRowB);
+    auto slot = [&](int row, int c) { return row * kRowB + ((c ^ (DH == 64 ? (row >> 1) & 7 : row & 15)) << 4); };
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq)
+        *reinterpret_cast<u32x2*>(ob + slot(col, 4 * db + rq) + 8 * hf) = quad(db, rq);
+    bf16_t* oh = out + (qrow + qw0) * DH;
+#pragma unroll
+    for (int p = 0; p < DH / 16; ++p) {
+      const int id = lane + 64 * p, row = id / (DH / 8), c = id % (DH / 8);
+      const u32x4 x = *reinterpret_cast<const u32x4*>(ob + slot(row, c));
+      if (qw0 + row < S) *reinterpret_cast<u32x4*>(oh + row * DH + 8 * c) = x;
+    }
   }
 }
 
