@@ -17,6 +17,7 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 from mlx_train_perf.errors import (
     AttentionInputError,
@@ -160,11 +161,13 @@ def nodes():
 
 
 def plain(*tensors: torch.Tensor) -> bool:
-    """Ordinary tensors outside function transforms, tracing and dispatch modes: the calls that the C++
-    nodes take. The others keep the Python Functions, which refuse or serve them as they always did."""
+    """Ordinary tensors outside function transforms, tracing and dispatch modes, without a forward-mode
+    tangent: the calls that the C++ nodes take. The others keep the Python Functions, which refuse or
+    serve them as they always did (a node sees no tangent of a tensor that is not its input)."""
     return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
             and not torch._C._are_functorch_transforms_active() and torch._C._get_tracing_state() is None
-            and not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0)
+            and not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
+            and (forward_ad._current_level < 0 or all(forward_ad.unpack_dual(t).tangent is None for t in tensors)))
 
 
 def gpu_available() -> bool:

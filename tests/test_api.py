@@ -267,3 +267,16 @@ def test_packed_layout_check_runs_again_after_in_place_edit():
     assert not api._layout_seen(pm)
     with pytest.raises(AttentionInputError):
         flash_attention(q, k, v, scale=1.0, impl="reference", segments=pm)
+
+
+def test_forward_mode_tangents_are_not_plain():
+    """Tensors with a forward-mode tangent do not go to the C++ nodes, which would drop it."""
+    from torch.autograd import forward_ad
+
+    from mlx_train_perf import _native
+
+    w, targets = torch.randn(4, 4), torch.arange(4)
+    assert _native.plain(w, targets)
+    with forward_ad.dual_level():
+        assert _native.plain(w, targets)
+        assert not _native.plain(w, targets, forward_ad.make_dual(w, torch.ones_like(w)))

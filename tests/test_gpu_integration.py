@@ -267,3 +267,41 @@ def test_loss_node_equals_the_python_function(kind, dtype, d, env, monkeypatch):
     assert node is not function and packed == packed_f
     assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
     L.clear_transposed_head_cache()
+
+
+@pytest.mark.parametrize("reduction", ["none", "mean", "sum"])
+@pytest.mark.parametrize("which", ["hidden", "trainable w", "frozen w", "scales", "biases"])
+def test_loss_refuses_forward_mode_tangents(which, reduction):
+    """No loss without its tangent: a dual tensor in any place is refused as the Python Function refuses it."""
+    from torch.autograd import forward_ad
+
+    from mlx_train_perf import DenseHead, QuantizedHead, linear_cross_entropy
+    from mlx_train_perf.core.quant import quantize
+
+    g = torch.Generator().manual_seed(3)
+    hidden, w = (torch.randn(n, 64, generator=g).to("cuda", torch.bfloat16) for n in (40, 300))
+    t = torch.randint(0, 300, (40,), generator=g).cuda()
+    q = dict(zip(("w_q", "scales", "biases"), quantize(w)))
+    with forward_ad.dual_level():
+        def dual(x):
+            return forward_ad.make_dual(x, torch.ones_like(x))
+
+        if which in q:
+            head = QuantizedHead(**{**q, which: dual(q[which])})
+        else:
+            head = DenseHead(weight=dual(w) if which.endswith("w") else w, trainable=which == "trainable w")
+        with pytest.raises(NotImplementedError):
+            linear_cross_entropy(dual(hidden) if which == "hidden" else hidden, head, t, reduction=reduction)
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+def test_attention_refuses_forward_mode_tangents(which):
+    from torch.autograd import forward_ad
+
+    from mlx_train_perf.attention import flash_attention
+
+    x = {n: torch.randn(1, 2, 32, 64, device="cuda", dtype=torch.bfloat16) for n in "qkv"}
+    with forward_ad.dual_level():
+        x[which] = forward_ad.make_dual(x[which], torch.ones_like(x[which]))
+        with pytest.raises(NotImplementedError):
+            flash_attention(**x, scale=0.125)
