@@ -143,7 +143,8 @@ struct KernelAttention : torch::autograd::Function<KernelAttention> {
   }
 };
 
-// A call of the loss beyond the hidden states and a trainable head's weight (its inputs).
+// A call of the loss. Its inputs are those of _KernelLCE that may ask for a gradient (also where they get none,
+// as a frozen weight does): hidden, w, scales, biases and the head's own weight, owner.
 struct LossCall {
   at::Tensor targets, w, w_q, scales, biases, owner;
   int64_t head_kind, fwd_kind, fwd_ws_bytes, ignore_index, bwd_chunk;
@@ -164,7 +165,8 @@ size_t budget_bytes() {
 
 struct KernelLoss : torch::autograd::Function<KernelLoss> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& hidden,
-                            const std::optional<at::Tensor>& trainable, const LossCall& c) {
+                            const std::optional<at::Tensor>& w, const std::optional<at::Tensor>& /*scales*/,
+                            const std::optional<at::Tensor>& /*biases*/, const at::Tensor& /*owner*/, const LossCall& c) {
     const c10::DeviceGuard device(hidden.device());
     const int64_t n = hidden.size(0), d = hidden.size(1), v = c.head_kind == MTP_HEAD_DENSE ? c.w.size(0) : c.w_q.size(0);
     const bool f32 = hidden.scalar_type() == at::kFloat;
@@ -207,7 +209,7 @@ struct KernelLoss : torch::autograd::Function<KernelLoss> {
     sd["head_kind"] = c.head_kind;
     sd["ignore_index"] = c.ignore_index;
     sd["bwd_chunk"] = c.bwd_chunk;
-    sd["d_w"] = trainable.has_value() && trainable->requires_grad();
+    sd["d_w"] = w.has_value() && w->requires_grad();
     ctx->set_materialize_grads(false);
     return out;
   }
@@ -248,7 +250,7 @@ struct KernelLoss : torch::autograd::Function<KernelLoss> {
                             opt_ptr<float>(biases), t, n, d, v, kind, ignore_index, ptr<float>(lse), ptr<float>(d_nll),
                             ptr<float>(d_hidden), opt_ptr<float>(d_w), chunk, ptr(ws), bytes, stream_of(hidden)),
             "loss");
-      return {d_hidden, d_w, at::Tensor()};
+      return {d_hidden, d_w, {}, {}, {}, {}};
     }
     // The head and workspace plan of _KernelLCE.backward; the cached transposed copies are the Python
     // layer's.
@@ -278,7 +280,7 @@ struct KernelLoss : torch::autograd::Function<KernelLoss> {
                         v, kind, ignore_index, ptr<float>(lse), ptr<float>(d_nll), ptr(d_hidden), opt_ptr(d_w), chunk, rows,
                         ptr(ws), bytes, stream_of(hidden)),
           "loss");
-    return {d_hidden, d_w, at::Tensor()};
+    return {d_hidden, d_w, {}, {}, {}, {}};
   }
 };
 
@@ -302,7 +304,7 @@ at::Tensor loss(const at::Tensor& hidden, const at::Tensor& targets, const std::
   const LossCall call{targets, w.value_or(none), w_q.value_or(none), scales.value_or(none), biases.value_or(none), owner,
                       head_kind, fwd_kind, fwd_ws_bytes, ignore_index, bwd_chunk, mean};
   return apply_node([&] {
-    return KernelLoss::apply(hidden, w.has_value() && w->requires_grad() ? w : std::nullopt, call);
+    return KernelLoss::apply(hidden, w, scales, biases, owner, call);
   });
 }
 

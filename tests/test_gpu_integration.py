@@ -305,3 +305,32 @@ def test_attention_refuses_forward_mode_tangents(which):
         x[which] = forward_ad.make_dual(x[which], torch.ones_like(x[which]))
         with pytest.raises(NotImplementedError):
             flash_attention(**x, scale=0.125)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("which", ["frozen w", "scales", "biases"])
+def test_loss_node_keeps_inputs_without_gradients_in_the_graph(which, dtype):
+    """A frozen weight, scales or biases that ask for a gradient are inputs of the loss, as they are of the
+    Python Function: the loss asks for one although hidden does not, and their accumulation hooks run (with
+    no gradient)."""
+    from mlx_train_perf import DenseHead, QuantizedHead, linear_cross_entropy
+    from mlx_train_perf.core.quant import quantize
+
+    g = torch.Generator().manual_seed(4)
+    hidden, w = (torch.randn(n, 64, generator=g).to("cuda", dtype) for n in (40, 300))
+    t = torch.randint(0, 300, (40,), generator=g).cuda()
+    q = dict(zip(("w_q", "scales", "biases"), quantize(w)))
+    x = (w if which == "frozen w" else q[which]).requires_grad_(True)
+    head = DenseHead(weight=w, trainable=False) if which == "frozen w" else QuantizedHead(**q)
+    calls = []
+    x.register_post_accumulate_grad_hook(lambda p: calls.append(p.grad))
+    for h in (hidden, hidden.clone().requires_grad_(True)):
+        for reduction in ("none", "mean", "sum"):
+            calls.clear()
+            loss = linear_cross_entropy(h, head, t, reduction=reduction)
+            assert loss.requires_grad
+            loss.sum().backward()
+            assert calls == [None] and x.grad is None
+            assert (h.grad is not None) == h.requires_grad
+    with torch.no_grad():
+        assert not linear_cross_entropy(hidden, head, t).requires_grad
