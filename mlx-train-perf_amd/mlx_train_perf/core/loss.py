@@ -493,13 +493,22 @@ def kernel_forward_parts(hidden2: torch.Tensor, head: HeadRef, targets2: torch.T
     return _KernelLCE.apply(*args, int(ignore_index), int(bwd_chunk or 0), owner)
 
 
+def _int64(x) -> bool:
+    """x is a whole number of 64 bits: what the node and the mean's kernels compare the targets with. The
+    others (torch compares with any number) keep the Python Function and torch's mean."""
+    return int(x) == x and -2 ** 63 <= x < 2 ** 63
+
+
 def _kernel_loss(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *, ignore_index: int,
                  bwd_chunk: int | None, mean: bool) -> torch.Tensor:
     """nll, or its mean over the tokens that are not ignored: the C++ node of _KernelLCE on plain tensors."""
-    *args, owner = _kernel_args(hidden2, head, targets2)
-    args += [int(ignore_index), int(bwd_chunk or 0), owner, mean]
-    h, _, w, w_q, _, _, kind = args[:7]
-    if not _native.plain(*(x for x in args if isinstance(x, torch.Tensor))):
+    *inputs, owner = _kernel_args(hidden2, head, targets2)
+    # A chunk of any size above the vocabulary is the whole vocabulary, one below a tile a tile; the node
+    # counts in 64 bits.
+    chunk = max(-1, min(int(bwd_chunk or 0), 2 ** 31))
+    args = (*inputs, int(ignore_index), chunk, owner, mean)
+    h, _, w, w_q, _, _, kind = inputs
+    if not (_int64(ignore_index) and _native.plain(*(x for x in args if isinstance(x, torch.Tensor)))):
         return _KernelLCE.apply(*args)[0]
     v, d = (w if kind == _native.HEAD_DENSE else w_q).shape[0], h.shape[1]
     ws_bytes = _forward_stage_bytes(_native.load(), h.shape[0], d, v, kind, h.dtype == torch.float32)
@@ -535,8 +544,8 @@ def linear_cross_entropy(
     elif resolved == "chunked":
         nll = _chunked_nll(hidden2, head, targets2, ignore_index, _DEFAULT_CHUNK if chunk_size is None else chunk_size)
     else:
-        nll = _kernel_loss(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size,
-                           mean=reduction == "mean")
-        if reduction == "mean":
+        mean = reduction == "mean" and _int64(ignore_index)
+        nll = _kernel_loss(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size, mean=mean)
+        if mean:
             return nll
     return _reduce(nll, reduction=reduction, leading=leading, targets2=targets2, ignore_index=ignore_index)

@@ -334,3 +334,35 @@ def test_loss_node_keeps_inputs_without_gradients_in_the_graph(which, dtype):
             assert (h.grad is not None) == h.requires_grad
     with torch.no_grad():
         assert not linear_cross_entropy(hidden, head, t).requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_loss_arguments_past_64_bits(dtype):
+    """Any chunk above the vocabulary is the whole vocabulary and any below a tile one tile, bit for bit; an
+    ignore_index that no target can hold, or that is no whole number, is taken as torch's operators take it."""
+    import sys
+
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+
+    g = torch.Generator().manual_seed(6)
+    hidden, w = (torch.randn(n, 128, generator=g).to("cuda", dtype) for n in (300, 1000))
+    hidden.requires_grad_(True)
+    head = DenseHead(weight=w * 0.05, trainable=False)
+    t = torch.randint(0, 1000, (300,), generator=g).cuda()
+
+    def step(**kw):
+        loss = linear_cross_entropy(hidden, head, t, **kw)
+        return loss.detach(), *torch.autograd.grad(loss, hidden)
+
+    whole, tile = step(chunk_size=1000), step(chunk_size=1)
+    assert not torch.equal(whole[1], tile[1])   # another order of sums
+    for size, want in ((sys.maxsize, whole), (2 ** 70, whole), (-5, tile), (-2 ** 70, tile)):
+        assert all(torch.equal(a, b) for a, b in zip(step(chunk_size=size), want)), size
+    none, count = linear_cross_entropy(hidden, head, t, reduction="none"), torch.tensor(300.0, device="cuda")
+    for index in (2 ** 63, 2 ** 64 - 100):
+        assert torch.equal(linear_cross_entropy(hidden, head, t, reduction="none", ignore_index=index), none)
+    assert torch.equal(linear_cross_entropy(hidden, head, t, ignore_index=2 ** 63), none.sum() / count)
+    t[:3] = 3
+    got = linear_cross_entropy(hidden, head, t, ignore_index=3.5)   # read as 3 by the loss, no target's equal
+    none = linear_cross_entropy(hidden, head, t, reduction="none", ignore_index=3)
+    assert torch.equal(got, none.sum() / count)
