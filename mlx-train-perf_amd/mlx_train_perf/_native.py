@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -131,33 +132,40 @@ def load() -> ctypes.CDLL:
         return lib
 
 
-_nodes = None
+_nodes = None   # the module once loaded, False where it cannot be
 
 
 def nodes():
     """Load (once) and return the extension module with the autograd nodes (csrc/torch_nodes.cpp), bound to
-    the loaded library's entry points; raise if it is absent."""
+    the loaded library's entry points. None where it was not built, or (with a warning) where it does not
+    load, as when it was built against another torch: the Python Functions then serve every call, the same
+    bits for more host time."""
     global _nodes
-    if _nodes is not None:
-        return _nodes
-    lib = load()
-    with _lock:
-        if _nodes is None:
-            try:
-                from mlx_train_perf import _mtp_torch
-            except ImportError as e:
-                raise MissingDependencyError(
-                    f"the autograd nodes {Path(__file__).with_name('_mtp_torch.so')} cannot be loaded ({e}); run "
-                    "`python -c \"import __graft_entry__ as g; g.build()\"` from the repository root.") from e
-            from mlx_train_perf.attention import api
-            from mlx_train_perf.core import loss
-            from mlx_train_perf.plan import launch
+    if _nodes is None:
+        lib = load()
+        with _lock:
+            if _nodes is None:
+                _nodes = _bind_nodes(lib)
+    return _nodes or None
 
-            _mtp_torch.bind({name: ctypes.cast(getattr(lib, name), _c_void_p).value for name in SIGNATURES}, check)
-            _mtp_torch.bind_attention(api.VJP_CALLS)
-            _mtp_torch.bind_loss(loss.VJP_CALLS, loss._transposed_head, launch.lce_bwd_budget_bytes)
-            _nodes = _mtp_torch
-    return _nodes
+
+def _bind_nodes(lib):
+    try:
+        from mlx_train_perf import _mtp_torch
+    except ImportError as e:
+        path = Path(__file__).with_name("_mtp_torch.so")
+        if path.exists():
+            warnings.warn(f"{path} cannot be loaded ({e}); calls take the Python autograd functions. Run "
+                          "`python -c \"import __graft_entry__ as g; g.build()\"` from the repository root.", stacklevel=2)
+        return False
+    from mlx_train_perf.attention import api
+    from mlx_train_perf.core import loss
+    from mlx_train_perf.plan import launch
+
+    _mtp_torch.bind({name: ctypes.cast(getattr(lib, name), _c_void_p).value for name in SIGNATURES}, check)
+    _mtp_torch.bind_attention(api.VJP_CALLS)
+    _mtp_torch.bind_loss(loss.VJP_CALLS, loss._transposed_head, launch.lce_bwd_budget_bytes)
+    return _mtp_torch
 
 
 def plain(*tensors: torch.Tensor) -> bool:

@@ -248,11 +248,11 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale:
                                       validate_segments=validate_segments)
     seg_id, seg_start = (None, None) if segments is None else _seg_args(q, segments.seg_id, segments.seg_start)
     if resolved == "kernel":
-        if _native.plain(q, k, v):
-            return _native.nodes().attention(q.contiguous(), k.contiguous(), v.contiguous(), seg_id, seg_start,
-                                             float(scale), bool(causal))
-        o, _ = _KernelAttention.apply(q.contiguous(), k.contiguous(), v.contiguous(), seg_id, seg_start, float(scale),
-                                      bool(causal))
+        args = (q.contiguous(), k.contiguous(), v.contiguous(), seg_id, seg_start, float(scale), bool(causal))
+        nodes = _native.nodes() if _native.plain(q, k, v) else None
+        if nodes is not None:
+            return nodes.attention(*args)
+        o, _ = _KernelAttention.apply(*args)
         return o
     o, _ = _ReferenceAttention.apply(q, k, v, seg_id, seg_start, float(scale), causal)
     return o

@@ -508,11 +508,13 @@ def _kernel_loss(hidden2: torch.Tensor, head: HeadRef, targets2: torch.Tensor, *
     chunk = max(-1, min(int(bwd_chunk or 0), 2 ** 31))
     args = (*inputs, int(ignore_index), chunk, owner, mean)
     h, _, w, w_q, _, _, kind = inputs
-    if not (_int64(ignore_index) and _native.plain(*(x for x in args if isinstance(x, torch.Tensor)))):
+    plain = _int64(ignore_index) and _native.plain(*(x for x in args if isinstance(x, torch.Tensor)))
+    nodes = _native.nodes() if plain else None
+    if nodes is None:
         return _KernelLCE.apply(*args)[0]
     v, d = (w if kind == _native.HEAD_DENSE else w_q).shape[0], h.shape[1]
     ws_bytes = _forward_stage_bytes(_native.load(), h.shape[0], d, v, kind, h.dtype == torch.float32)
-    return _native.nodes().loss(*args, _native.HEAD_Q4_STAGED if ws_bytes else kind, ws_bytes)
+    return nodes.loss(*args, _native.HEAD_Q4_STAGED if ws_bytes else kind, ws_bytes)
 
 
 def linear_cross_entropy(

@@ -280,3 +280,26 @@ def test_forward_mode_tangents_are_not_plain():
     with forward_ad.dual_level():
         assert _native.plain(w, targets)
         assert not _native.plain(w, targets, forward_ad.make_dual(w, torch.ones_like(w)))
+
+
+def test_missing_autograd_nodes_are_remembered(monkeypatch):
+    """Without the extension module nodes() is None, asked once, and a file that does not load says so."""
+    import sys
+    import warnings
+    from pathlib import Path
+
+    import mlx_train_perf
+    from mlx_train_perf import _native
+
+    monkeypatch.setattr(_native, "_nodes", None)
+    monkeypatch.delattr(mlx_train_perf, "_mtp_torch", raising=False)
+    monkeypatch.setitem(sys.modules, "mlx_train_perf._mtp_torch", None)   # its import fails
+    monkeypatch.setattr(Path, "exists", lambda self: True)
+    with pytest.warns(UserWarning, match="cannot be loaded"):
+        assert _native.nodes() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.nodes() is None
+        monkeypatch.setattr(_native, "_nodes", None)
+        monkeypatch.setattr(Path, "exists", lambda self: self.suffix != ".so" or "libmtp" in self.name)
+        assert _native.nodes() is None   # not built: no warning

@@ -366,3 +366,32 @@ def test_loss_arguments_past_64_bits(dtype):
     got = linear_cross_entropy(hidden, head, t, ignore_index=3.5)   # read as 3 by the loss, no target's equal
     none = linear_cross_entropy(hidden, head, t, reduction="none", ignore_index=3)
     assert torch.equal(got, none.sum() / count)
+
+
+def test_calls_without_the_autograd_nodes(monkeypatch):
+    """An installation with the C-ABI library alone: the Python Functions serve every call, the same bits."""
+    import sys
+
+    import mlx_train_perf
+    from mlx_train_perf import DenseHead, _native, linear_cross_entropy
+    from mlx_train_perf.attention import flash_attention
+
+    g = torch.Generator().manual_seed(8)
+    x, w = (torch.randn(n, 64, generator=g).to("cuda", torch.bfloat16).requires_grad_(True) for n in (40, 300))
+    q = torch.randn(1, 2, 70, 64, generator=g).to("cuda", torch.bfloat16).requires_grad_(True)
+    t = torch.randint(0, 300, (40,), generator=g).cuda()
+
+    def calls():
+        loss = linear_cross_entropy(x, DenseHead(weight=w), t)
+        o = flash_attention(q, q, q, scale=0.125)
+        grads = torch.autograd.grad(loss, (x, w)) + torch.autograd.grad(o.float().square().sum(), q)
+        return (loss.detach(), o.detach(), *grads), (type(loss.grad_fn).__name__, type(o.grad_fn).__name__)
+
+    want, built = calls()
+    monkeypatch.setattr(_native, "_nodes", None)
+    monkeypatch.delattr(mlx_train_perf, "_mtp_torch", raising=False)
+    monkeypatch.setitem(sys.modules, "mlx_train_perf._mtp_torch", None)   # its import fails
+    with pytest.warns(UserWarning, match="cannot be loaded"):
+        got, names = calls()
+    assert names == ("_KernelLCEBackward", "_KernelAttentionBackward") and not set(names) & set(built)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
