@@ -29,6 +29,7 @@
 extern "C" {
 #endif
 
+/* Raised when a declaration below changes or goes. New exports may join a version. */
 #define MTP_ABI_VERSION 5
 
 /* Error codes; the Python layer maps them onto the reference's typed exceptions

@@ -121,13 +121,16 @@ def load() -> ctypes.CDLL:
                 "g.build()\"` from the repository root (hipcc --offload-arch=gfx950)."
             )
         lib = ctypes.CDLL(str(LIB_PATH), mode=ctypes.RTLD_GLOBAL)
+        version = lib.mtp_abi_version() if hasattr(lib, "mtp_abi_version") else None
+        if version != ABI_VERSION:
+            raise MissingDependencyError(f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
+        missing = [name for name in SIGNATURES if not hasattr(lib, name)]
+        if missing:   # an older build of this version, which grows by new exports
+            raise MissingDependencyError(f"{LIB_PATH} does not export {', '.join(missing)}; rebuild it")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        if lib.mtp_abi_version() != ABI_VERSION:
-            raise MissingDependencyError(f"{LIB_PATH} has ABI version {lib.mtp_abi_version()}, expected "
-                                         f"{ABI_VERSION}; rebuild it")
         _lib = lib
         return lib
 

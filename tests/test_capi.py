@@ -12,6 +12,7 @@ from hypothesis import given, settings
 from hypothesis import strategies as st
 
 from mlx_train_perf import _native
+from mlx_train_perf.errors import MissingDependencyError
 from mlx_train_perf.plan import launch as plan
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -90,6 +91,23 @@ def test_library_exports_every_declared_symbol():
         assert hasattr(lib, name), name
     assert set(_native.SIGNATURES) >= declared - set()  # every export has a Python signature
     assert lib.mtp_abi_version() == _native.ABI_VERSION == 5
+
+
+@pytest.mark.parametrize(("source", "what"), [
+    ("int mtp_abi_version(void) { return 5; }", "does not export mtp_last_error"),   # an older build of the version
+    ("int mtp_abi_version(void) { return 4; }", "ABI version 4"), ("int unrelated(void) { return 5; }", "ABI version None")])
+def test_a_library_that_does_not_fit_is_refused_with_its_reason(source, what, tmp_path, monkeypatch):
+    import shutil
+    import subprocess
+
+    if shutil.which("gcc") is None:
+        pytest.skip("no C compiler")
+    path = tmp_path / "libold.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", "-", "-o", str(path)], input=source.encode(), check=True)
+    monkeypatch.setattr(_native, "LIB_PATH", path)
+    monkeypatch.setattr(_native, "_lib", None)
+    with pytest.raises(MissingDependencyError, match=what):
+        _native.load()
 
 
 @pytest.mark.parametrize(("n", "d", "v"), [(8192, 4096, 151936), (1024, 512, 32000), (65, 192, 1027), (1, 8, 1),
