@@ -36,6 +36,10 @@ from mlx_train_perf.plan import launch as _plan
 _KERNEL_DTYPES = (torch.bfloat16, torch.float32)
 _KERNEL_ROW_TILE = 256  # token rows per workgroup tile (reported as Resolution.row_tiles)
 _DEFAULT_CHUNK = 8192   # chunked-impl vocab chunk (the reference's kernel tile, loss.py:25)
+# Tokens up to which the mean runs in the loss's own node (mtp_lce_mean, one workgroup). Mean and its gradient on
+# the GPU, against torch's operators: 5 / 22 us at 8192 tokens, 14 / 35 at 65536, 25 / 34 at 131072,
+# 46 / 34 at 262144, 290 / 39 at 1048576.
+_MEAN_TOKENS = 131072
 _WORD_DTYPES = tuple(t for t in (torch.int32, getattr(torch, "uint32", None)) if t is not None)
 
 
@@ -546,7 +550,7 @@ def linear_cross_entropy(
     elif resolved == "chunked":
         nll = _chunked_nll(hidden2, head, targets2, ignore_index, _DEFAULT_CHUNK if chunk_size is None else chunk_size)
     else:
-        mean = reduction == "mean" and _int64(ignore_index)
+        mean = reduction == "mean" and hidden2.shape[0] <= _MEAN_TOKENS and _int64(ignore_index)
         nll = _kernel_loss(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size, mean=mean)
         if mean:
             return nll

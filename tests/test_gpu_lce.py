@@ -223,6 +223,31 @@ def test_mean_loss_and_its_gradient(n, ignored):
     assert torch.equal(dh, ref)
 
 
+@pytest.mark.parametrize(("past", "own"), [(0, True), (1, False)])
+def test_mean_of_many_tokens(past, own):
+    """Up to _MEAN_TOKENS the mean is the loss's own node; past them torch's operators, whose time does not grow
+    with one workgroup's. Both against the mean in 64 bits."""
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+    from mlx_train_perf.core import loss as L
+
+    n = L._MEAN_TOKENS + past
+    g = torch.Generator().manual_seed(n)
+    h = torch.randn(n, 8, generator=g).to("cuda", torch.bfloat16).requires_grad_(True)
+    w = torch.randn(9, 8, generator=g).to("cuda", torch.bfloat16)
+    t = torch.randint(0, 9, (n,), generator=g).cuda()
+    t[::5] = IGN
+    head = DenseHead(weight=w, trainable=False)
+    loss = linear_cross_entropy(h, head, t)
+    assert ("Div" not in type(loss.grad_fn).__name__) is own
+    nll = linear_cross_entropy(h, head, t, reduction="none")
+    want = float(nll.detach().double().sum() / (t != IGN).sum())
+    # one rounding of the 64-bit mean; of torch's fp32 sum n roundings, at random (sqrt(n))
+    assert abs(float(loss.detach()) - want) <= (2 ** -23 if own else n ** 0.5 * 2 ** -24) * want
+    (dh,) = torch.autograd.grad(loss, h)
+    (ref,) = torch.autograd.grad(nll, h, torch.ones_like(nll) / (t != IGN).sum())
+    assert torch.equal(dh, ref)
+
+
 def test_undefined_gradient_is_zero():
     """A user's autograd node that returns no gradient for the losses or for O: the gradients are zeros."""
     from mlx_train_perf import DenseHead, linear_cross_entropy
