@@ -2107,9 +2107,8 @@ hipError_t launch_lce_fwd(const LceHead& h, const bf16_t* H, const int64_t* targ
 
 // Mean loss of the tokens that are not ignored: mean = sum(nll) / max(count, 1), summed in 64 bits (an
 // ignored token's nll is 0), and the count. One workgroup, bound by its loads: 3.6 us at 8192 tokens
-// (96 KiB), 12.5 at 65536, 23 at 131072, 285 at 1048576; as torch operators (compare, two sums, clamp,
-// convert, divide) it is six launches, 19 us at 8192, 31 at 131072, 36 at 1048576. The loss layer asks
-// for it up to 131072 tokens.
+// (96 KiB), 12.5 at 65536, 285 at 1048576; as torch operators (compare, two sums, clamp, convert, divide) it
+// is six launches, 19 us at 8192, 31 at 65536, 36 at 1048576. The loss layer asks for it up to 98304 tokens.
 __global__ __launch_bounds__(1024) void lce_mean_kernel(const float* __restrict__ nll,
                                                         const int64_t* __restrict__ targets, long n,
                                                         long long ignore_index, float* __restrict__ mean,

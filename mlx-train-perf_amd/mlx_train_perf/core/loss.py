@@ -36,10 +36,10 @@ from mlx_train_perf.plan import launch as _plan
 _KERNEL_DTYPES = (torch.bfloat16, torch.float32)
 _KERNEL_ROW_TILE = 256  # token rows per workgroup tile (reported as Resolution.row_tiles)
 _DEFAULT_CHUNK = 8192   # chunked-impl vocab chunk (the reference's kernel tile, loss.py:25)
-# Tokens up to which the mean runs in the loss's own node (mtp_lce_mean, one workgroup). Mean and its gradient on
-# the GPU, against torch's operators: 5 / 22 us at 8192 tokens, 14 / 35 at 65536, 25 / 34 at 131072,
-# 46 / 34 at 262144, 290 / 39 at 1048576.
-_MEAN_TOKENS = 131072
+# Tokens up to which the mean runs in the loss's own node (mtp_lce_mean, one workgroup). What the mean adds to a
+# forward (D = 64, V = 1000), against torch's operators: 20 / 37 us at 65536 tokens, 31 / 49 at 98304, 40 / 36 at
+# 131072; alone 43 / 31 at 262144 and 285 / 36 at 1048576.
+_MEAN_TOKENS = 98304
 _WORD_DTYPES = tuple(t for t in (torch.int32, getattr(torch, "uint32", None)) if t is not None)
 
 
