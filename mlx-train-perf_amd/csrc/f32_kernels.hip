@@ -845,8 +845,8 @@ void attn32_q_kernel(const float* __restrict__ q, const float* __restrict__ k, c
   f32x4 acc[L::kB];
 #pragma unroll
   for (int i = 0; i < L::kB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  ln.copy(kh, kv_begin, S, lds0, true);
-  ln.copy(vh, kv_begin, S, lds0 + L::kTile, true);
+  ln.copy(kh, kv_begin, S, lds0, ntiles > 0);  // no tile (a segment start past the queries): nothing read
+  ln.copy(vh, kv_begin, S, lds0 + L::kTile, ntiles > 0);
   copies_landed();
   // The row loads are complete here: tell the compiler, which would wait for them (and for the copies
   // in flight) at their first use.

@@ -211,6 +211,24 @@ def test_attention_fp32_block_edges(shape, mask):
     _attn_check(got, q, k, v, do, scale, causal=mask != "full", sid=sid, tag=f"{shape} {mask}")
 
 
+@pytest.mark.parametrize("d", [64, 96, 128])
+def test_attention_fp32_segment_start_past_the_row(d):
+    """Unchecked segments that start past every query (past the row, too) leave it no key: nothing is read for
+    it, zeros and L = -inf come out, as from the bf16 kernels."""
+    from mlx_train_perf.attention.api import kernel_backward, kernel_forward
+
+    b, h, s = 1, 2, 70
+    q, k, v, do = (torch.randn(b, h, s, d, device="cuda") for _ in range(4))
+    for start in (s - 1, s, 10 * s):
+        sid = torch.zeros(b, s, dtype=torch.int32, device="cuda")
+        sst = torch.full((b, s), start, dtype=torch.int32, device="cuda")
+        none = torch.arange(s, device="cuda") < start   # the last query sees itself when start = s - 1
+        o, lse = kernel_forward(q, k, v, scale=0.1, seg_id=sid, seg_start=sst)
+        assert not o[:, :, none].any() and (lse[:, :, none] == -math.inf).all()
+        dq, _, _ = kernel_backward(q, k, v, o, lse, do, scale=0.1, seg_id=sid, seg_start=sst)
+        assert not dq[:, :, none].any()
+
+
 def test_attention_fp32_workspace_for_d_alone_runs_unsplit():
     """mtp_attn_bwd_f32 with room for D only gives the split pass's gradients, summed in another order."""
     from mlx_train_perf import _native
