@@ -170,6 +170,14 @@ int mtp_lce_bwd(const void* hidden, const void* w, const void* w_t, const uint32
                 const float* d_nll, void* d_hidden, void* d_w, int64_t chunk, int64_t row_block,
                 void* workspace, size_t workspace_bytes, void* stream);
 
+/* reduction="mean" of the forward's per-token loss (fp32 [n]; 0 for ignored tokens): mean = sum(nll) /
+ * max(count, 1) with count the tokens whose target is not ignore_index (both one float on the device), and
+ * its gradient d_nll[i] = d_mean / count. No reference counterpart (the reference has no ignore_index; its
+ * trainer adapter divides by ntoks, adapters/mlx_lm.py:212-216). */
+int mtp_lce_mean(const float* nll, const int64_t* targets, int64_t n, int64_t ignore_index, float* mean,
+                 float* count, void* stream);
+int mtp_lce_mean_bwd(const float* d_mean, const float* count, int64_t n, float* d_nll, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * (B) Flash attention. Layouts (attention/reference.py:22-25): q [b][hq][s][dh],
  * k, v [b][hkv][s][dh], o like q, lse fp32 [b][hq][s] (natural log). GQA: query head h reads
@@ -183,14 +191,6 @@ int mtp_lce_bwd(const void* hidden, const void* w, const void* w_t, const uint32
  * attention (causal = 0: every key visible to every query; an extension -- the reference kernel
  * serves causal only and refuses causal=False, api.py:109-113). Segments require causal = 1.
  * ------------------------------------------------------------------------------------------- */
-
-/* reduction="mean" of the forward's per-token loss (fp32 [n]; 0 for ignored tokens): mean = sum(nll) /
- * max(count, 1) with count the tokens whose target is not ignore_index (both one float on the device), and
- * its gradient d_nll[i] = d_mean / count. No reference counterpart (the reference has no ignore_index; its
- * trainer adapter divides by ntoks, adapters/mlx_lm.py:212-216). */
-int mtp_lce_mean(const float* nll, const int64_t* targets, int64_t n, int64_t ignore_index, float* mean,
-                 float* count, void* stream);
-int mtp_lce_mean_bwd(const float* d_mean, const float* count, int64_t n, float* d_nll, void* stream);
 
 /* Forward: o = softmax(scale * q k^T + mask) v, lse = row logsumexp of the masked scaled scores.
  * Replaces: launch_flash_fwd (attention/kernel/launch.py:386-441) + kernel K7

@@ -1,8 +1,9 @@
 // fp32 inputs: the fused linear cross-entropy and flash attention for fp32 hidden states / q, k, v
 // (the reference kernels take fp32 as well as bf16: core/loss.py:24, attention/api.py:41-43).
 //
-// Arithmetic is fp32 end to end: v_mfma_f32_32x32x2_f32 products (exact fp32 multiplies, fp32
-// accumulation), fp32 softmax statistics, fp32 outputs and gradients. The algorithms are those of
+// Arithmetic is fp32 end to end: fp32 MFMA products (exact fp32 multiplies, fp32 accumulation;
+// v_mfma_f32_32x32x2_f32 in the LCE, v_mfma_f32_16x16x4_f32 in attention), fp32 softmax statistics,
+// fp32 outputs and gradients. The algorithms are those of
 // the bf16 kernels (lce_kernels.hip, attn_kernels.hip) and of the reference's oracles:
 //   LCE forward: per token lse = logsumexp_v(h . w_v) (online over vocab tiles, vocab splits merged
 //     by the finalize), tgt = h . w_y, nll = lse - tgt (core/naive.py:9-14, core/chunked.py:35-49);
@@ -13,12 +14,10 @@
 //     query-head group (attention/reference.py:37-116, attention/api.py:126-194).
 //
 // MFMA 32x32x2 f32 lane layout (wave64): lane l supplies A[i = l % 32][k = l / 32] and
-// B[k = l / 32][j = l % 32]; its 16 results are C[i = 8 (r / 4) + 4 (l / 32) + r % 4][j = l % 32].
-// A 16-deep contraction chunk runs as 8 MFMAs in which lane half h contracts k = 8 h + s at step s,
-// so each lane reads 8 consecutive k of its row (two 16-byte LDS reads). In the products whose
-// contraction index is the row index of an accumulator (P V, dS K, ...), step s pairs keys
-// 8 (s / 4) + 4 h + s % 4, the keys register r = s of the accumulator holds, so the probability and
-// dS registers feed the next product directly.
+// B[k = l / 32][j = l % 32]; its 16 results are C[i = 8 (r / 4) + 4 (l / 32) + r % 4][j = l % 32]. Which k a
+// lane half contracts at which step is each core's choice (both operands make the same), so that a lane
+// reads consecutive k of its row: the register-staged core k = 8 h + s of 16, the copied one
+// 8 c + 4 h + s of 32. The 16x16x4 layout stands at the attention kernels.
 #include "mtp_common.hpp"
 #include "mtp_launch.hpp"
 
@@ -1121,8 +1120,9 @@ hipError_t launch_lce32_fwd(const LceHead32& h, const float* H, const int64_t* t
 }
 
 // Contraction parts of the fp32 dH product of a chunk of kcols columns: about two workgroups per
-// CU over the ceil(N/128) x ceil(D/128) output tiles, each part at least 512 columns (32 stages)
-// and a multiple of 16 (one stage); at most 32. *per receives the columns per part.
+// CU over the ceil(N/128) x ceil(D/128) output tiles, each part at least 512 columns (32 stages of the
+// register-staged core, 16 of the copied one) and a multiple of 16 (the copied core reads zeros past a
+// part's end); at most 32. *per receives the columns per part.
 int lce32_dh_parts(long N, long D, long kcols, int* per) {
   const long tiles = ((N + kT - 1) / kT) * ((D + kT - 1) / kT);
   long np = (2L * kNumCU + tiles - 1) / tiles;

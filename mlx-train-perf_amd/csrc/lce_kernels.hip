@@ -1283,7 +1283,6 @@ void lce_bwd_g_kernel(const bf16_t* __restrict__ H, const bf16_t* __restrict__ W
 constexpr int kGBlockBytes = 4096;   // a wave's staging block: 32 tokens x 64 columns
 constexpr int kGStores = 2 * 4 * kNJ;  // 16-byte stores per thread and tile
 
-
 __device__ __forceinline__ void store16(const u32x4& x, const __amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
   __builtin_amdgcn_raw_buffer_store_b128(x, r, voff, soff, 0);
 }
@@ -1343,6 +1342,7 @@ void lce_bwd_g_persist_kernel(const bf16_t* __restrict__ H, const bf16_t* __rest
                               int wrow0, bf16_t* __restrict__ G) {
   // One array: with a second one the compiler tracks the copies into LDS by array and waits for all
   // of them (vmcnt(0)) before fragment reads of every stage (flagship 4.09 -> 4.62 ms).
+  static_assert(kLdsBytes + (Q4 ? kQ4SbBytes : 8 * kGBlockBytes) <= 160 * 1024, "more than a CU's LDS");
   __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes + (Q4 ? kQ4SbBytes : 8 * kGBlockBytes)];
 
   const int g = blockIdx.x;
@@ -2205,7 +2205,7 @@ static hipError_t lce_bwd_rows(const LceHead& h, const bf16_t* H, const int64_t*
       }
     }
     if (D % kBK == 0) {
-      // One resident workgroup per CU (the stages take 128 KiB of LDS, 144 KiB for the 4-bit head).
+      // One resident workgroup per CU (160 KiB of LDS, all of it, with a dense head; 130 KiB with a 4-bit one).
       const int ns = lce_nsplit(N, (long)ctiles * kTile, 1);
       dim3 pgrid(rtiles * ns);
       if (gq4) {

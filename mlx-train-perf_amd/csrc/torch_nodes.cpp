@@ -1,11 +1,12 @@
 // The autograd nodes of flash_attention and linear_cross_entropy on plain tensors: the forward and backward of
-// attention/api.py's _KernelAttention and core/loss.py's _KernelLCE without the interpreter in the backward.
-// Autograd runs a backward on a thread of its own; a Python node there waits for the interpreter lock and
-// pulls the interpreter's state to that thread's core, and the next forward pulls it back, which doubles
-// the host time of both. Forward and backward of an attention layer (B = 4, S = 509, 16/8 heads,
-// head_dim 64, 55 us of kernels): 124 us with the Python node, 79 with this one; of a small mean loss
-// (N = 128, D = 256, V = 3000, 106 us of kernels): 179 and 133. The entry points of the C-ABI library come from
-// the Python layer (bind), so both use the one it loaded.
+// attention/api.py's _KernelAttention and core/loss.py's _KernelLCE, planned and launched from C++.
+// Autograd runs a backward on a thread of its own; a Python node there holds the interpreter lock for the
+// whole of it and pulls the interpreter's state to that thread's core, and the next forward pulls it back.
+// A node here takes the lock for a moment: once to count the backward, and in a loss also for the workspace
+// budget and the cached transposed head. A pass of an attention layer (B = 4, S = 509, 16/8 heads, head_dim 64)
+// takes 75 or 122 us with the Python node, 45 or 78 with this one, by where the thread lands; of a small mean
+// loss (N = 128, D = 256, V = 3000) 165 us, and 65 or 110. The entry points of the C-ABI library come from the
+// Python layer (bind), so both use the one it loaded.
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>

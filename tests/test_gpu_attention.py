@@ -89,9 +89,9 @@ def test_causal_parity_edge_lengths(shape):
             assert rel_l2(got, want) <= 1e-2
 
 
-# Workgroups of the dK/dV pass with 0 to 6 tiles: up to 40 (head, 64-query tile) items over 8 splits. Its loop
+# Workgroups of the dK/dV pass with 0 to 8 tiles: up to 60 (head, 64-query tile) items over 8 splits. Its loop
 # runs three tiles at a time and finishes the last one by itself.
-@pytest.mark.parametrize("s", [64, 130, 257, 385, 449, 600])
+@pytest.mark.parametrize("s", [64, 130, 257, 385, 449, 600, 700, 900])
 @pytest.mark.parametrize("causal", [True, False])
 def test_dkv_tile_counts(s, causal):
     q, k, v, do = attn_inputs(1, 4, 1, s, 64, seed=s)

@@ -191,8 +191,8 @@ def test_attention_fp32_parity(shape, causal):
 
 
 # Edges of the 16-query and 16-key waves, of the 32-position tiles, of the 64-key blocks and of the pairs of
-# blocks (odd and even counts, one block alone) for workgroups of 4, 2 and 1 heads; the last with enough
-# items for 16 splits of the dK/dV pass.
+# blocks (odd and even counts, one block alone) for workgroups of 4, 2 and 1 heads, with 1 to 16 splits of
+# the dK/dV pass.
 @pytest.mark.parametrize("shape", [(1, 4, 1, 15, 64), (1, 2, 1, 16, 96), (1, 3, 3, 17, 128), (2, 6, 2, 31, 64),
                                    (1, 4, 4, 33, 96), (1, 8, 1, 64, 128), (1, 2, 2, 65, 64), (1, 4, 2, 129, 96),
                                    (1, 3, 1, 192, 128), (1, 4, 1, 513, 64)])

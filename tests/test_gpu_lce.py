@@ -514,10 +514,8 @@ def test_backward_many_vocab_tiles_per_workgroup(n, d, v, head):
     assert row.max() <= 2.0 ** -7
 
 
-# (n, d, v, chunk, head): one chunk and several (the last one partial), a split dH contraction
-# (n = 1000, d = 2048), a tiny grid and a 256-column chunk; 4-bit and dense heads.
 # The 64 x 64-tile dH product (a vocabulary of up to 15 tiles): row counts around its tiles and its 512
-# workgroups, one to three slabs per wave, several chunks (its fp32 accumulator), and the first sizes past it.
+# workgroups, none to eight slabs per wave, several chunks (its fp32 accumulator), and the first sizes past it.
 @pytest.mark.parametrize(("n", "d", "v", "chunk"), [(1, 64, 1, None), (64, 128, 256, None), (65, 192, 1000, 256),
                                                     (200, 64, 3840, None), (130, 320, 3841, None), (257, 256, 1100, 512),
                                                     (1024, 2048, 500, None), (1025, 2048, 500, None)])
@@ -543,6 +541,8 @@ def test_backward_small_output_tiles(n, d, v, chunk, head):
     assert rel_l2(hd.grad.cpu(), odh.cpu()) <= 1e-2 or (v == 1 and float(hd.grad.float().norm()) < 1e-3)
 
 
+# (n, d, v, chunk, head): one chunk and several (the last one partial), a split dH contraction
+# (n = 1000, d = 2048), a tiny grid and a 256-column chunk; 4-bit and dense heads.
 @pytest.mark.parametrize(("n", "d", "v", "chunk", "head"), [(1000, 512, 6000, 2048, "q4"),
                                                             (1000, 2048, 8000, 8192, "q4"),
                                                             (300, 256, 3000, 256, "q4"),
