@@ -550,7 +550,10 @@ def linear_cross_entropy(
     elif resolved == "chunked":
         nll = _chunked_nll(hidden2, head, targets2, ignore_index, _DEFAULT_CHUNK if chunk_size is None else chunk_size)
     else:
-        mean = reduction == "mean" and hidden2.shape[0] <= _MEAN_TOKENS and _int64(ignore_index)
+        # (a captured graph keeps the node's: torch's sum over many blocks clears memory by a memset node, which
+        # has given wrong values on later replays)
+        mean = (reduction == "mean" and _int64(ignore_index)
+                and (hidden2.shape[0] <= _MEAN_TOKENS or torch.cuda.is_current_stream_capturing()))
         nll = _kernel_loss(hidden2, head, targets2, ignore_index=ignore_index, bwd_chunk=chunk_size, mean=mean)
         if mean:
             return nll

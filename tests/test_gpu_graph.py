@@ -160,3 +160,37 @@ def test_packed_attention_step_replays_in_a_hip_graph():
         torch.cuda.synchronize()
         for name, a, e in zip(("O", "dQ", "dK", "dV"), got, (oe.detach(), qe.grad, ke.grad, ve.grad)):
             assert torch.equal(a, e), f"replay {rep} ({lens}): {name}"
+
+
+def test_mean_of_many_tokens_replays_in_a_hip_graph():
+    """Past the tokens up to which the loss's own mean is the faster one, a captured step keeps it: its mean is
+    the 64-bit one rounded once on every replay (torch's multi-block sum would record a memset node)."""
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+    from mlx_train_perf.core import loss as L
+
+    n = L._MEAN_TOKENS + 1
+    g0 = torch.Generator().manual_seed(2)
+    head = DenseHead(weight=torch.randn(9, 8, generator=g0).to("cuda", torch.bfloat16), trainable=False)
+    hs = torch.randn(n, 8, generator=g0).to("cuda", torch.bfloat16).requires_grad_(True)
+    ts = torch.randint(0, 9, (n,), generator=g0).cuda()
+
+    def step():
+        loss = linear_cross_entropy(hs, head, ts, validate_targets=False)
+        return (loss, *torch.autograd.grad(loss, hs))
+
+    g, (loss, dh) = _capture(step)
+    for _ in range(4):
+        with torch.no_grad():
+            hs.copy_(torch.randn(n, 8, generator=g0).cuda())
+        ts.copy_(torch.randint(0, 9, (n,), generator=g0).cuda())
+        ts[::3] = -100
+        g.replay()
+        torch.cuda.synchronize()
+        got, got_dh = float(loss), dh.clone()
+        _eager_work()
+        nll = linear_cross_entropy(hs, head, ts, reduction="none")
+        count = (ts != -100).sum()
+        want = float(nll.detach().double().sum() / count)
+        assert abs(got - want) <= 2 ** -23 * want
+        (ref,) = torch.autograd.grad(nll, hs, torch.ones(n, device="cuda") / count)
+        assert torch.equal(got_dh, ref)
