@@ -71,7 +71,6 @@ def build(verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as ex:
         nodes = ex.submit(_build_nodes)
         objs = list(ex.map(_compile, SOURCES))
-        nodes.result()
     tmp = OUT.with_suffix(".so.tmp")
     # --no-undefined: a kernel whose host launch stub was not emitted fails here, not at load time.
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,--no-undefined", "-o", str(tmp), *map(str, objs)]
@@ -79,6 +78,7 @@ def build(verbose: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, OUT)
+    nodes.result()   # raises with the library in place: it serves every call without them
     if verbose:
         print(f"built {OUT} and {NODE_OUT.name}")
     return OUT

@@ -303,3 +303,28 @@ def test_missing_autograd_nodes_are_remembered(monkeypatch):
         monkeypatch.setattr(_native, "_nodes", None)
         monkeypatch.setattr(Path, "exists", lambda self: self.suffix != ".so" or "libmtp" in self.name)
         assert _native.nodes() is None   # not built: no warning
+
+
+def test_build_leaves_the_library_where_the_nodes_fail(monkeypatch, tmp_path):
+    """Without a host compiler or Python's headers the nodes do not build: build() says so, after the library,
+    which serves every call without them."""
+    import subprocess
+    from pathlib import Path
+
+    from mlx_train_perf import _build
+
+    def link(cmd, **kw):
+        Path(cmd[cmd.index("-o") + 1]).touch()
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    def nodes():
+        raise RuntimeError("no Python.h")
+
+    monkeypatch.setattr(_build, "OUT", tmp_path / "libmtp_hip.so")
+    monkeypatch.setattr(_build, "OBJ_DIR", tmp_path / "obj")
+    monkeypatch.setattr(_build, "_compile", lambda src: tmp_path / src)
+    monkeypatch.setattr(_build, "_build_nodes", nodes)
+    monkeypatch.setattr(_build.subprocess, "run", link)
+    with pytest.raises(RuntimeError, match="no Python.h"):
+        _build.build()
+    assert (tmp_path / "libmtp_hip.so").exists()
