@@ -14,8 +14,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
-#include <cstdlib>
-#include <cstring>
+#include <string>
 
 #include "../../include/mtp_hip.h"
 
@@ -46,12 +45,13 @@ struct Entries {
 Entries g_api;
 // Python: the typed error of a return code (_native.check), the call counters of the attention and the
 // loss (VJP_CALLS), the loss layer's cache of transposed heads (_transposed_head) and its workspace budget
-// (plan.launch.lce_bwd_budget_bytes). Held until the process ends.
+// (plan.launch.lce_bwd_budget_bytes), os.environ.get. Held until the process ends.
 PyObject* g_check = nullptr;
 PyObject* g_attn_calls = nullptr;
 PyObject* g_lce_calls = nullptr;
 PyObject* g_transposed_head = nullptr;
 PyObject* g_budget = nullptr;
+PyObject* g_env = nullptr;
 
 void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
@@ -152,9 +152,13 @@ struct LossCall {
   bool mean;
 };
 
+// A switch of the environment as Python sees it (C's getenv may not run beside another thread's setenv).
 bool env_is(const char* name, const char* value) {
-  const char* e = std::getenv(name);
-  return e != nullptr && std::strcmp(e, value) == 0;
+  return python([&] {
+    const py::handle get(g_env);
+    const py::object x = get(name);
+    return !x.is_none() && x.cast<std::string>() == value;
+  });
 }
 
 size_t budget_bytes() {
@@ -344,10 +348,11 @@ void bind(const py::dict& entries, py::object check_fn) {
   g_check = check_fn.release().ptr();
 }
 void bind_attention(py::object calls) { g_attn_calls = calls.release().ptr(); }
-void bind_loss(py::object calls, py::object transposed_head, py::object budget) {
+void bind_loss(py::object calls, py::object transposed_head, py::object budget, py::object env) {
   g_lce_calls = calls.release().ptr();
   g_transposed_head = transposed_head.release().ptr();
   g_budget = budget.release().ptr();
+  g_env = env.release().ptr();
 }
 
 }  // namespace

@@ -167,7 +167,7 @@ def _bind_nodes(lib):
 
     _mtp_torch.bind({name: ctypes.cast(getattr(lib, name), _c_void_p).value for name in SIGNATURES}, check)
     _mtp_torch.bind_attention(api.VJP_CALLS)
-    _mtp_torch.bind_loss(loss.VJP_CALLS, loss._transposed_head, launch.lce_bwd_budget_bytes)
+    _mtp_torch.bind_loss(loss.VJP_CALLS, loss._transposed_head, launch.lce_bwd_budget_bytes, os.environ.get)
     return _mtp_torch
 
 

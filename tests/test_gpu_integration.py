@@ -395,3 +395,22 @@ def test_calls_without_the_autograd_nodes(monkeypatch):
         got, names = calls()
     assert names == ("_KernelLCEBackward", "_KernelAttentionBackward") and not set(names) & set(built)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_loss_node_reads_the_environment_as_python_does():
+    """A switch set in the C environment alone (os.putenv) is none to os.environ, nor to the node's backward."""
+    import os
+
+    from mlx_train_perf import DenseHead, linear_cross_entropy
+    from mlx_train_perf.core import loss as L
+
+    assert "MTP_LCE_TRANSPOSED_HEAD" not in os.environ
+    g = torch.Generator().manual_seed(5)
+    x, w = (torch.randn(n, 64, generator=g).to("cuda", torch.bfloat16).requires_grad_(True) for n in (40, 300))
+    L.clear_transposed_head_cache()
+    os.putenv("MTP_LCE_TRANSPOSED_HEAD", "1")   # would keep a trainable head's transposed copy
+    try:
+        linear_cross_entropy(x, DenseHead(weight=w), torch.zeros(40, dtype=torch.int64, device="cuda")).backward()
+    finally:
+        os.unsetenv("MTP_LCE_TRANSPOSED_HEAD")
+    assert L.transposed_head_cache_bytes() == 0
